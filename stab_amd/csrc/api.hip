@@ -603,7 +603,9 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
   if (lds > 160 * 1024) return fail(c, STAB_E_ARG, "operator workspace %zu B exceeds LDS", lds);
   HIPCHECK(c, hipMemsetAsync(B.state, 0, sizeof(KSState) * npts, c->stream));
   const cx<T> *mats = (const cx<T> *)B.mats, *blks = (const cx<T> *)B.blks;
-  const size_t lds_schur = sizeof(zd) * (2 * kp.m * kp.m + kp.m + KS_NEVMAX * kp.m);
+  int nevmax = 1;
+  for (const auto &d : B.h) nevmax = std::max(nevmax, d.nev);
+  const size_t lds_schur = schur_lds_bytes(kp.m, nevmax);
   std::vector<KSState> hs(npts);
   cycles_max = 0;
   ms_arnoldi = 0.0;
@@ -618,7 +620,7 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
                          B.pivs, blks, B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax,
                          B.nymax, B.nvecmax, cyc == 0 ? 1 : 0);
     HIPCHECK(c, hipEventRecord(c->ev[6], c->stream));
-    hipLaunchKernelGGL(k_schur, dim3(npts), dim3(64), lds_schur, c->stream, B.pts, B.small, B.state, kp.m, kp.keep,
+    hipLaunchKernelGGL(k_schur, dim3(npts), dim3(128), lds_schur, c->stream, B.pts, B.small, B.state, kp.m, kp.keep,
                        kp.tol);
     HIPCHECK(c, hipGetLastError());
     HIPCHECK(c, hipMemcpyAsync(hs.data(), B.state, sizeof(KSState) * npts, hipMemcpyDeviceToHost, c->stream));

@@ -509,234 +509,396 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 3
 }
 
 // ---------------------------------------------------------------------------
-// Small dense eigenproblem of H_m (one wave): Householder reduction to
-// Hessenberg form, complex single-shift QR to Schur form T = Q^H H Q, then the
-// `keep` eigenvalues of largest modulus are moved to the leading positions in
+// Small dense eigenproblem of H_m: Householder reduction to Hessenberg form,
+// complex single-shift QR to Schur form T = Q^H H Q, then the `keep`
+// eigenvalues of largest modulus are moved to the leading positions in
 // decreasing modulus.  Ritz vectors of the first nev, residual estimates and
 // convergence are written back.
+//
+// One work-group of two waves per point: wave 0 works on H, wave 1 applies the
+// rotations of each finished sweep to Q while wave 0 runs the next (two
+// rotation lists, one barrier a sweep).  The step is a chain of some 2500
+// dependent rotations (m = 40), so what counts is the latency of one.  A sweep
+// therefore runs in two phases.  Lane j owns column j while the rotations are
+// found: it carries its entry of the current row in a register and reads the
+// next row ahead, and the 3 x 3 window that determines the next rotation is
+// held by every lane, so no rotation waits for LDS.  Then lane i owns row i
+// and applies the sweep's rotations to the columns in one pass.  With a lone
+// wave, LDS round trips and library hypot calls in every rotation a point
+// took 2.95 ms (m = 40) and 1.09 ms (m = 24); this form takes 1.21 and 0.52 ms,
+// some 780 cycles a rotation in phase 1 (about 55 FP64 operations, mostly
+// dependent) and 220 in phase 2.
 // ---------------------------------------------------------------------------
-__device__ inline void givens(zd x, zd y, double &c, zd &s) {
-  const double ax = cabs(x), ay = cabs(y);
-  if (ay == 0.0) { c = 1.0; s = czero<double>(); return; }
-  if (ax == 0.0) { c = 0.0; s = conj(y) * (1.0 / ay); return; }
-  const double r = hypot(ax, ay);
-  c = ax / r;
-  s = (x * (1.0 / ax)) * conj(y) * (1.0 / r);
+// Order LDS accesses of one wave's lanes (a wave's LDS operations execute in
+// order; this keeps the compiler to it).
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ inline double lane_get(double x, int l) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)(unsigned int)(b & 0xffffffffLL), l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
+}
+__device__ inline zd lane_get(zd x, int l) { return mk(lane_get(x.x, l), lane_get(x.y, l)); }
+// Sum over the wave, in every lane (row shifts, then row broadcasts; lanes
+// without a source add nothing).
+template <int CTRL, int RM> __device__ inline double dpp_or_zero(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b & 0xffffffffLL), CTRL, RM, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RM, 0xF, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
+}
+__device__ inline double wave_sum(double x) {
+  x += dpp_or_zero<0x111, 0xF>(x);
+  x += dpp_or_zero<0x112, 0xF>(x);
+  x += dpp_or_zero<0x114, 0xF>(x);
+  x += dpp_or_zero<0x118, 0xF>(x);
+  x += dpp_or_zero<0x142, 0xA>(x);
+  x += dpp_or_zero<0x143, 0xC>(x);
+  return lane63(x);
 }
 
-__global__ __launch_bounds__(64) void k_schur(const PointDev *__restrict__ pts, zd *__restrict__ small,
-                                              KSState *__restrict__ st, int m, int keep, double tol) {
+// Rotation with c x + s y = r, c y - conj(s) x = 0, c real, the same (x, y) in
+// every lane.  Squares that would under- or overflow, and x = 0, take the
+// scaled form.
+__device__ inline void givens(zd x, zd y, double &c, zd &s) {
+  const double x2 = abs2(x), n2 = x2 + abs2(y);
+  const double rx = rsqrt(x2), f = rx * rsqrt(n2);
+  c = x2 * f;
+  s = x * conj(y) * f;
+  if (__builtin_expect(!(x2 > 1e-280 && n2 < 1e280), 0)) {
+    const double big = fmax(fmax(fabs(x.x), fabs(x.y)), fmax(fabs(y.x), fabs(y.y)));
+    const int ex = -__builtin_amdgcn_frexp_exp(big);       // 0 for a big of 0, Inf or NaN
+    x = mk(ldexp(x.x, ex), ldexp(x.y, ex));
+    y = mk(ldexp(y.x, ex), ldexp(y.y, ex));
+    const double xs = abs2(x), ys = abs2(y);
+    const double r1 = xs == 0.0 ? 0.0 : rsqrt(xs), r2 = rsqrt(xs + ys);
+    c = ys == 0.0 ? 1.0 : xs * r1 * r2;
+    s = ys == 0.0 ? czero<double>() : (xs == 0.0 ? conj(y) * r2 : x * conj(y) * (r1 * r2));
+  }
+}
+
+struct Rot { double c; zd s; };
+
+// b when p, else a, by components (a ternary of structures selects between
+// addresses and sends both to scratch memory).
+__device__ inline zd sel(bool p, zd b, zd a) { return mk(p ? b.x : a.x, p ? b.y : a.y); }
+
+// a <- a R over columns (k, k + 1) for the rotation list r[k], k = k0 .. hi - 1
+// ascending (UP; k0 >= lo may differ from lane to lane) or k = hi - 1 .. lo
+// descending, on the row whose entry of column k is a[k ld].  Entries and
+// rotations are read four steps ahead.
+template <bool UP>
+__device__ inline void rotate_row(zd *a, int ld, const Rot *r, int lo, int hi, int k0) {
+  zd p = a[(size_t)(UP ? k0 : hi) * ld];
+  for (int b = 0; b < hi - lo; b += 4) {
+    zd q[4];
+    Rot g[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = UP ? min(lo + b + u, hi - 1) : max(hi - 1 - b - u, lo);
+      q[u] = a[(size_t)(UP ? k + 1 : k) * ld];
+      g[u] = r[k];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = UP ? lo + b + u : hi - 1 - b - u;
+      const double c = g[u].c;
+      const zd s = g[u].s;
+      if (UP) {
+        if (k >= k0 && k < hi) {
+          a[(size_t)k * ld] = p * c + conj(s) * q[u];
+          p = q[u] * c - s * p;
+        }
+      } else if (k >= lo) {            // p carries the column that moves left
+        a[(size_t)(k + 1) * ld] = p * c - s * q[u];
+        p = q[u] * c + conj(s) * p;
+      }
+    }
+  }
+  a[(size_t)(UP ? hi : lo) * ld] = p;
+}
+
+// sum_i conj(v_i) a[i ld] (CONJ) or sum_i a[i ld] v_i over i0 <= i < i1, four
+// entries' loads at a time.
+template <bool CONJ>
+__device__ inline zd strided_dot(const zd *a, int ld, const zd *v, int i0, int i1) {
+  zd s[2] = {czero<double>(), czero<double>()};
+  for (int i = i0; i < i1; i += 4) {
+    zd x[4], w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = min(i + u, i1 - 1);
+      x[u] = a[j * ld];
+      w[u] = v[j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i + u < i1) s[u & 1] = CONJ ? cfmac(s[u & 1], w[u], x[u]) : cfma(s[u & 1], x[u], w[u]);
+  }
+  return s[0] + s[1];
+}
+// a[i ld] -= s conj(v_i) (CONJ) or s v_i.
+template <bool CONJ>
+__device__ inline void strided_sub(zd *a, int ld, const zd *v, zd s, int i0, int i1) {
+  for (int i = i0; i < i1; i += 4) {
+    zd x[4], w[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = min(i + u, i1 - 1);
+      x[u] = a[j * ld];
+      w[u] = v[j];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (i + u < i1) a[(i + u) * ld] = cfms(x[u], s, CONJ ? conj(w[u]) : w[u]);
+  }
+}
+
+// LDS of k_schur: H (rows padded by one entry: lane i reading row i meets
+// distinct banks), Q column-major, two rotation lists (the Householder vector
+// and the triangular eigenvectors of the first nev use their space).
+__host__ __device__ inline size_t schur_lds_bytes(int m, int nevmax) {
+  const size_t work = sizeof(Rot) * 2 * m, zz = sizeof(zd) * nevmax * nevmax;
+  return sizeof(zd) * ((size_t)m * (m + 1) + (size_t)m * m) + (work > zz ? work : zz);
+}
+
+__global__ __launch_bounds__(128) void k_schur(const PointDev *__restrict__ pts, zd *__restrict__ small,
+                                               KSState *__restrict__ st, int m, int keep, double tol) {
   extern __shared__ zd sl[];
   const PointDev &P = pts[blockIdx.x];
   KSState S = st[blockIdx.x];
   if (S.done) return;
-  zd *Hs = sl, *Q = Hs + m * m, *v = Q + m * m, *zz = v + m;   // zz: KS_NEVMAX * m
+  const int LD = m + 1;
+  zd *Hs = sl, *Qs = Hs + m * LD;               // H(i, j) at Hs[i LD + j], Q(i, j) at Qs[j m + i]
+  Rot *rot = (Rot *)(Qs + m * m);               // list b at rot + b m
+  zd *v = (zd *)rot, *zz = (zd *)rot;
+  __shared__ int s_lo[2], s_hi[2];              // range of each list; s_hi < 0 ends a stage
+  __shared__ double s_est[KS_NEVMAX];
   zd *Hg = small + P.small_off + SM_H;
   zd *Qg = small + P.small_off + SM_Q;
   zd *Yg = small + P.small_off + SM_Y;
   zd *THg = small + P.small_off + SM_TH;
-  const int ldh = KS_MMAX + 1, t = threadIdx.x;
+  const int ldh = KS_MMAX + 1, t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int nev = P.nev;
-  for (int e = t; e < m * m; e += 64) {
+  for (int e = t; e < m * m; e += 128) {
     const int i = e % m, j = e / m;
-    Hs[i * m + j] = Hg[(size_t)j * ldh + i];   // row-major in LDS
-    Q[i * m + j] = (i == j) ? mk(1.0, 0.0) : czero<double>();
+    Hs[i * LD + j] = Hg[(size_t)j * ldh + i];
+    Qs[j * m + i] = (i == j) ? mk(1.0, 0.0) : czero<double>();
   }
   const zd hlast = Hg[(size_t)(m - 1) * ldh + m];
   __syncthreads();
-  // --- Householder reduction to Hessenberg form
+  // --- Householder reduction to Hessenberg form: v = x - alpha e1 with
+  // |v|^2 = 2 nx (nx + |x0|).  Both waves form the norms of column k.
   for (int k = 0; k < m - 2; ++k) {
     const int len = m - k - 1;
-    double nx = 0.0;
-    for (int i = 0; i < len; ++i) nx += abs2(Hs[(k + 1 + i) * m + k]);
-    double below = nx - abs2(Hs[(k + 1) * m + k]);
-    if (below <= 1e-300 * (nx + 1e-300)) continue;     // already reduced
-    nx = sqrt(nx);
-    const zd x0 = Hs[(k + 1) * m + k];
-    const double ax0 = cabs(x0);
+    const zd xi = (lane < len) ? Hs[(k + 1 + lane) * LD + k] : czero<double>();
+    const double nx2 = wave_sum(abs2(xi));
+    const zd x0 = lane_get(xi, 0);
+    const double below = nx2 - abs2(x0);
+    if (below <= 1e-300 * (nx2 + 1e-300)) continue;     // already reduced (the same in every lane)
+    const double nx = sqrt(nx2), ax0 = sqrt(abs2(x0));
     const zd ph = (ax0 > 0.0) ? x0 * (1.0 / ax0) : mk(1.0, 0.0);
-    const zd alpha = ph * (-nx);
-    // v = x - alpha e1, normalised
-    for (int i = t; i < len; i += 64) v[i] = (i == 0) ? x0 - alpha : Hs[(k + 1 + i) * m + k];
+    const double iv = rsqrt(2.0 * nx * (nx + ax0));
+    if (wv == 0 && lane < len) v[lane] = sel(lane == 0, x0 + ph * nx, xi) * iv;
     __syncthreads();
-    double vn = 0.0;
-    for (int i = 0; i < len; ++i) vn += abs2(v[i]);
-    vn = sqrt(vn);
-    __syncthreads();
-    for (int i = t; i < len; i += 64) v[i] = v[i] * (1.0 / vn);
-    __syncthreads();
-    // H <- (I - 2 v v^H) H  on rows k+1.., columns k..m-1
-    for (int c = k + t; c < m; c += 64) {
-      zd s = czero<double>();
-      for (int i = 0; i < len; ++i) s = cfmac(s, v[i], Hs[(k + 1 + i) * m + c]);
-      for (int i = 0; i < len; ++i) Hs[(k + 1 + i) * m + c] = cfms(Hs[(k + 1 + i) * m + c], v[i], s * 2.0);
+    // H <- (I - 2 v v^H) H on rows k+1.., columns k..m-1: a wave takes 32
+    // columns, half a wave each half of the rows
+    {
+      const int c = k + 32 * wv + (lane & 31), half = lane >> 5, mid = (len + 1) / 2;
+      const int i0 = half ? mid : 0, i1 = half ? len : mid;
+      zd *col = Hs + (k + 1) * LD + min(c, m - 1);
+      zd s = strided_dot<true>(col, LD, v, i0, i1);
+      s.x += __shfl_xor(s.x, 32);
+      s.y += __shfl_xor(s.y, 32);
+      if (c < m) strided_sub<false>(col, LD, v, s * 2.0, i0, i1);
     }
     __syncthreads();
-    // H <- H (I - 2 v v^H) on columns k+1.., all rows; Q likewise
-    for (int rr = t; rr < 2 * m; rr += 64) {
-      zd *row = (rr < m) ? &Hs[rr * m] : &Q[(rr - m) * m];
-      zd s = czero<double>();
-      for (int i = 0; i < len; ++i) s = cfma(s, row[k + 1 + i], v[i]);
-      for (int i = 0; i < len; ++i) row[k + 1 + i] = cfms(row[k + 1 + i], s * 2.0, conj(v[i]));
+    // H <- H (I - 2 v v^H) on columns k+1.. (wave 0, a row per lane), Q
+    // likewise (wave 1)
+    if (lane < m) {
+      zd *row = wv ? Qs + (size_t)(k + 1) * m + lane : Hs + lane * LD + k + 1;
+      const int ld = wv ? m : 1;
+      const zd s = strided_dot<false>(row, ld, v, 0, len);
+      strided_sub<true>(row, ld, v, s * 2.0, 0, len);
     }
-    __syncthreads();
-    if (t == 0)
-      for (int i = 2; i < len + 1; ++i) Hs[(k + i) * m + k] = czero<double>();
+    if (wv == 0) {
+      wave_lds_fence();
+      if (lane >= 1 && lane < len) Hs[(k + 1 + lane) * LD + k] = czero<double>();
+    }
     __syncthreads();
   }
-  // --- complex QR iterations to Schur form (full T and Q)
+  // --- complex QR sweeps to Schur form (full T and Q); pass n fills list n & 1
   const double eps = 2.220446049250313e-16;
-  int hi = m - 1, iter = 0, total = 0;
-  while (hi > 0 && total < 60 * m) {
-    int lo = hi;
-    while (lo > 0) {
-      const double sub = cabs1(Hs[lo * m + lo - 1]);
-      const double dia = cabs1(Hs[lo * m + lo]) + cabs1(Hs[(lo - 1) * m + lo - 1]);
-      if (sub <= eps * dia || sub < 1e-300) break;
-      --lo;
-    }
-    if (lo > 0) {
-      __syncthreads();
-      if (t == 0) Hs[lo * m + lo - 1] = czero<double>();
-      __syncthreads();
-    }
-    if (lo == hi) { --hi; iter = 0; continue; }
-    ++iter; ++total;
-    zd mu;
-    const zd a = Hs[(hi - 1) * m + hi - 1], b = Hs[(hi - 1) * m + hi], c = Hs[hi * m + hi - 1], d = Hs[hi * m + hi];
-    if (iter % 11 == 10) {
-      mu = d + mk(0.75 * cabs(c), 0.0);
-    } else {
-      const zd half = (a - d) * 0.5;
-      zd disc = half * half + b * c;
-      // complex sqrt
-      const double r = cabs(disc);
-      double sr = sqrt(0.5 * (r + fabs(disc.x)));
-      zd sq;
-      if (sr == 0.0) sq = czero<double>();
-      else if (disc.x >= 0) sq = mk(sr, disc.y / (2.0 * sr));
-      else sq = mk(fabs(disc.y) / (2.0 * sr), disc.y >= 0 ? sr : -sr);
-      const zd m1 = (a + d) * 0.5 + sq, m2 = (a + d) * 0.5 - sq;
-      mu = (cabs(m1 - d) < cabs(m2 - d)) ? m1 : m2;
-    }
-    for (int k = lo; k < hi; ++k) {
-      zd x, y;
-      if (k == lo) { x = Hs[lo * m + lo] - mu; y = Hs[(lo + 1) * m + lo]; }
-      else { x = Hs[k * m + k - 1]; y = Hs[(k + 1) * m + k - 1]; }
-      double cg; zd sg;
-      givens(x, y, cg, sg);
-      __syncthreads();
-      const int c0 = (k > lo) ? k - 1 : lo;
-      for (int jj = c0 + t; jj < m; jj += 64) {
-        const zd p = Hs[k * m + jj], q = Hs[(k + 1) * m + jj];
-        Hs[k * m + jj] = p * cg + sg * q;
-        Hs[(k + 1) * m + jj] = q * cg - conj(sg) * p;
+  if (wv == 0) {
+    int hi = m - 1, iter = 0, total = 0, n = 0;
+    while (hi > 0 && total < 60 * m) {
+      // negligible subdiagonals of the active part, all at once
+      bool neg = false;
+      if (lane >= 1 && lane <= hi) {
+        const double sub = cabs1(Hs[lane * LD + lane - 1]);
+        const double dia = cabs1(Hs[lane * LD + lane]) + cabs1(Hs[(lane - 1) * LD + lane - 1]);
+        neg = sub <= eps * dia || sub < 1e-300;
       }
-      __syncthreads();
-      const int rmax = min(k + 2, hi);
-      for (int ii = t; ii <= rmax; ii += 64) {
-        const zd p = Hs[ii * m + k], q = Hs[ii * m + k + 1];
-        Hs[ii * m + k] = p * cg + conj(sg) * q;
-        Hs[ii * m + k + 1] = q * cg - sg * p;
+      const unsigned long long negm = __ballot(neg);
+      while (hi > 0 && ((negm >> hi) & 1ull)) {
+        if (lane == 0) Hs[hi * LD + hi - 1] = czero<double>();
+        --hi;
+        iter = 0;
       }
-      for (int ii = t; ii < m; ii += 64) {
-        const zd p = Q[ii * m + k], q = Q[ii * m + k + 1];
-        Q[ii * m + k] = p * cg + conj(sg) * q;
-        Q[ii * m + k + 1] = q * cg - sg * p;
+      if (hi == 0) break;
+      const unsigned long long below = negm & ((1ull << hi) - 1ull);
+      const int lo = below ? 63 - __builtin_clzll(below) : 0;
+      if (lo > 0 && lane == 0) Hs[lo * LD + lo - 1] = czero<double>();
+      wave_lds_fence();
+      ++iter;
+      ++total;
+      zd mu;
+      const zd a = Hs[(hi - 1) * LD + hi - 1], b = Hs[(hi - 1) * LD + hi], c = Hs[hi * LD + hi - 1], d = Hs[hi * LD + hi];
+      if (iter % 11 == 10) {
+        mu = d + mk(0.75 * sqrt(abs2(c)), 0.0);
+      } else {
+        const zd half = (a - d) * 0.5;
+        const zd disc = half * half + b * c;
+        const double r = sqrt(abs2(disc)), sr = sqrt(0.5 * (r + fabs(disc.x)));
+        zd sq;
+        if (sr == 0.0) sq = czero<double>();
+        else if (disc.x >= 0) sq = mk(sr, disc.y / (2.0 * sr));
+        else sq = mk(fabs(disc.y) / (2.0 * sr), disc.y >= 0 ? sr : -sr);
+        const zd m1 = (a + d) * 0.5 + sq, m2 = (a + d) * 0.5 - sq;
+        mu = (abs2(m1 - d) < abs2(m2 - d)) ? m1 : m2;
       }
+      // phase 1, lane j = column j.  At rotation k (rows k, k + 1): e = row k,
+      // h = row k + 1, hn = row k + 2, hnn = row k + 3 of the lane's column.
+      // Columns > k have met no column rotation yet; those of columns k - 1
+      // and k are applied to e and h of lanes k - 1 and k as they are found,
+      // so one row rotation serves every lane.  (x, y) = e, h of lane k - 1.
+      Rot *rl = rot + (n & 1) * m;
+      const int col = min(lane, m - 1);
+      zd e = Hs[lo * LD + col], h = Hs[(lo + 1) * LD + col], hn = Hs[min(lo + 2, hi) * LD + col];
+      zd x = lane_get(e, lo) - mu, y = lane_get(h, lo);
+      for (int k = lo; k < hi; ++k) {
+        const zd hnn = Hs[min(k + 3, hi) * LD + col];     // past hi: not used
+        const zd G = lane_get(hn, k + 1);
+        double cg;
+        zd sg;
+        givens(x, y, cg, sg);
+        const zd sc = conj(sg);
+        if (lane == 0) { rl[k].c = cg; rl[k].s = sg; }
+        const zd f = e * cg + sg * h;
+        e = h * cg - sc * e;
+        if (lane < m && lane >= (k > lo ? k - 1 : k)) Hs[k * LD + lane] = f;
+        // the column rotation (k, k + 1) on rows k + 1 and k + 2
+        const zd C1 = lane_get(e, k), D1 = lane_get(e, k + 1);
+        x = C1 * cg + sc * D1;
+        y = sc * G;
+        e = sel(lane == k, x, sel(lane == k + 1, D1 * cg - sg * C1, e));
+        h = sel(lane == k, y, sel(lane == k + 1, G * cg, hn));
+        hn = hnn;
+      }
+      if (lane < m && lane >= hi - 1) Hs[hi * LD + lane] = e;
+      wave_lds_fence();
+      // phase 2, lane i = row i: the sweep's column rotations from max(lo, i) on
+      // (those before met row i inside the window)
+      if (lane < hi) rotate_row<true>(Hs + lane * LD, 1, rl, lo, hi, max(lo, lane));
+      wave_lds_fence();
+      if (lane == 0) { s_lo[n & 1] = lo; s_hi[n & 1] = hi; }
+      ++n;
+      __syncthreads();       // list n - 1 is complete; wave 1 is done with the other one
+    }
+    if (lane == 0) s_hi[n & 1] = -1;
+    __syncthreads();
+  } else {
+    for (int n = 0;; ++n) {
       __syncthreads();
-      if (k > lo && t == 0) Hs[(k + 1) * m + k - 1] = czero<double>();
-      __syncthreads();
+      const int lo = s_lo[n & 1], hi = s_hi[n & 1];
+      if (hi < 0) break;
+      if (lane < m) rotate_row<true>(Qs + lane, m, rot + (n & 1) * m, lo, hi, lo);
     }
   }
   __syncthreads();
-  // --- reorder: bring the `keep` eigenvalues of largest modulus to the front
-  for (int pos = 0; pos < keep; ++pos) {
-    int best = pos;
-    double bv = cabs(Hs[pos * m + pos]);
-    for (int i = pos + 1; i < m; ++i) {
-      const double vv = cabs(Hs[i * m + i]);
-      if (vv > bv) { bv = vv; best = i; }
+  // --- reorder: bring the `keep` eigenvalues of largest modulus to the front;
+  // pass pos fills list pos & 1 (an empty range when nothing moves)
+  if (wv == 0) {
+    for (int pos = 0; pos < keep; ++pos) {
+      const double av = (lane >= pos && lane < m) ? sqrt(abs2(Hs[min(lane, m - 1) * LD + min(lane, m - 1)])) : -1.0;
+      double bv = av;
+      for (int off = 32; off > 0; off >>= 1) bv = fmax(bv, __shfl_xor(bv, off));
+      const unsigned long long at = __ballot(av == bv);
+      const int best = at ? max(pos, __builtin_ctzll(at)) : pos;   // NaN entries compare unequal
+      Rot *rl = rot + (pos & 1) * m;
+      const zd t22 = Hs[best * LD + best];                          // the eigenvalue that moves up
+      for (int k = best - 1; k >= pos; --k) {
+        const zd t11 = Hs[k * LD + k];
+        double cg;
+        zd sg;
+        givens(Hs[k * LD + k + 1], t22 - t11, cg, sg);
+        if (lane == 0) { rl[k].c = cg; rl[k].s = sg; }
+        const int jj = k + lane;
+        if (jj < m) {
+          const zd p = Hs[k * LD + jj], q = Hs[(k + 1) * LD + jj];
+          Hs[k * LD + jj] = p * cg + sg * q;
+          Hs[(k + 1) * LD + jj] = q * cg - conj(sg) * p;
+        }
+        wave_lds_fence();
+        if (lane <= k + 1) {
+          const zd p = Hs[lane * LD + k], q = Hs[lane * LD + k + 1];
+          // rows k and k + 1 of the 2 x 2 block are known: [t22, .; 0, t11]
+          Hs[lane * LD + k] = sel(lane == k, t22, sel(lane == k + 1, czero<double>(), p * cg + conj(sg) * q));
+          Hs[lane * LD + k + 1] = sel(lane == k + 1, t11, q * cg - sg * p);
+        }
+        wave_lds_fence();
+      }
+      if (lane == 0) { s_lo[pos & 1] = pos; s_hi[pos & 1] = best; }
+      __syncthreads();
     }
-    for (int k = best - 1; k >= pos; --k) {
-      const zd t11 = Hs[k * m + k], t22 = Hs[(k + 1) * m + k + 1];
-      double cg; zd sg;
-      givens(Hs[k * m + k + 1], t22 - t11, cg, sg);
+  } else {
+    for (int pos = 0; pos < keep; ++pos) {
       __syncthreads();
-      for (int jj = k + t; jj < m; jj += 64) {
-        const zd p = Hs[k * m + jj], q = Hs[(k + 1) * m + jj];
-        Hs[k * m + jj] = p * cg + sg * q;
-        Hs[(k + 1) * m + jj] = q * cg - conj(sg) * p;
-      }
-      __syncthreads();
-      for (int ii = t; ii <= k + 1; ii += 64) {
-        const zd p = Hs[ii * m + k], q = Hs[ii * m + k + 1];
-        Hs[ii * m + k] = p * cg + conj(sg) * q;
-        Hs[ii * m + k + 1] = q * cg - sg * p;
-      }
-      for (int ii = t; ii < m; ii += 64) {
-        const zd p = Q[ii * m + k], q = Q[ii * m + k + 1];
-        Q[ii * m + k] = p * cg + conj(sg) * q;
-        Q[ii * m + k + 1] = q * cg - sg * p;
-      }
-      __syncthreads();
-      if (t == 0) {
-        Hs[k * m + k] = t22;
-        Hs[(k + 1) * m + k + 1] = t11;
-        Hs[(k + 1) * m + k] = czero<double>();
-      }
-      __syncthreads();
+      if (lane < m && s_hi[pos & 1] > pos) rotate_row<false>(Qs + lane, m, rot + (pos & 1) * m, pos, s_hi[pos & 1], 0);
     }
   }
-  // --- eigenvectors of T for the first nev (lane i handles pair i)
+  __syncthreads();
+  // --- eigenvectors of T for the first nev (thread i handles pair i; entries
+  // past i vanish)
   if (t < nev) {
     const int i = t;
-    zd *z = zz + i * m;
-    const zd ti = Hs[i * m + i];
+    zd *z = zz + i * nev;
+    const zd ti = Hs[i * LD + i];
     const double smin = fmax(eps * cabs(ti), 1e-300);
-    for (int l = 0; l < m; ++l) z[l] = czero<double>();
     z[i] = mk(1.0, 0.0);
     for (int l = i - 1; l >= 0; --l) {
       zd s = czero<double>();
-      for (int c = l + 1; c <= i; ++c) s = cfma(s, Hs[l * m + c], z[c]);
-      zd d = Hs[l * m + l] - ti;
+      for (int c = l + 1; c <= i; ++c) s = cfma(s, Hs[l * LD + c], z[c]);
+      zd d = Hs[l * LD + l] - ti;
       if (cabs(d) < smin) d = mk(smin, 0.0);
       z[l] = czero<double>() - cdiv(s, d);
     }
   }
   __syncthreads();
-  // y_i = Q z_i, normalised; residual estimate |h_{m,m-1}| |y_i[m-1]|
-  __shared__ double s_est[KS_NEVMAX];
-  if (t < nev) {
-    const int i = t;
-    const zd *z = zz + i * m;
-    double nn = 0.0;
-    zd ylast = czero<double>();
-    for (int r = 0; r < m; ++r) {
-      zd s = czero<double>();
-      for (int c = 0; c <= i; ++c) s = cfma(s, Q[r * m + c], z[c]);
-      nn += abs2(s);
-      if (r == m - 1) ylast = s;
-    }
-    const double inv = 1.0 / sqrt(nn);
-    for (int r = 0; r < m; ++r) {
-      zd s = czero<double>();
-      for (int c = 0; c <= i; ++c) s = cfma(s, Q[r * m + c], z[c]);
-      Yg[(size_t)i * KS_MMAX + r] = s * inv;
-    }
-    const zd th = Hs[i * m + i];
-    s_est[i] = cabs(hlast) * cabs(ylast) * inv / fmax(cabs(th), 1e-300);
+  // y_i = Q z_i, normalised (a wave per pair, a row per lane); residual
+  // estimate |h_{m,m-1}| |y_i[m-1]|
+  for (int i = wv; i < nev; i += 2) {
+    const zd *z = zz + i * nev;
+    zd s = czero<double>();
+    if (lane < m)
+      for (int c = 0; c <= i; ++c) s = cfma(s, Qs[c * m + lane], z[c]);
+    const double inv = 1.0 / sqrt(wave_sum(abs2(s)));
+    if (lane < m) Yg[(size_t)i * KS_MMAX + lane] = s * inv;
+    if (lane == m - 1) s_est[i] = cabs(hlast) * cabs(s) * inv / fmax(cabs(Hs[i * LD + i]), 1e-300);
   }
-  __syncthreads();
-  // write T (row-major -> column-major global H) and Q, theta
-  for (int e = t; e < m * m; e += 64) {
+  // write Q (the kept columns), theta and T
+  for (int e = t; e < m * keep; e += 128) {
     const int i = e % m, j = e / m;
-    Qg[(size_t)j * KS_MMAX + i] = Q[i * m + j];
+    Qg[(size_t)j * KS_MMAX + i] = Qs[j * m + i];
   }
-  for (int i = t; i < m; i += 64) THg[i] = Hs[i * m + i];
-  for (int e = t; e < keep * keep; e += 64) {
+  for (int i = t; i < m; i += 128) THg[i] = Hs[i * LD + i];
+  for (int e = t; e < keep * keep; e += 128) {
     const int i = e % keep, j = e / keep;
-    Hg[(size_t)j * ldh + i] = (i <= j) ? Hs[i * m + j] : czero<double>();
+    Hg[(size_t)j * ldh + i] = (i <= j) ? Hs[i * LD + j] : czero<double>();
   }
   __syncthreads();
   if (t == 0) {
