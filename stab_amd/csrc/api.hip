@@ -588,9 +588,21 @@ int run_graph(stab_ctx *c, const std::vector<long long> &sig, F issue, int *how)
   return STAB_OK;
 }
 
+// Work-group size of the iteration kernels (k_arnoldi, k_invit, k_final) for
+// `active` points: one wide work-group per point while that leaves CUs without
+// any (lu_solve_wide), four waves beyond, where two or three work-groups share
+// a CU and memory is the bound.  STAB_WIDE_POINTS moves the line.
+// Krylov leading modes, N = 96, four waves against wide, ms: 14.1 / 11.1 at 64
+// points, 23.6 / 20.1 at 256, 32.5 / 27.4 at 320, 27.1 / 26.3 at 512, 51.3 /
+// 50.4 at 1024; inverse iteration 7.1 / 6.8 at 64, 7.1 / 7.1 at 256, 8.3 / 8.6
+// at 320, 15.1 / 15.3 at 1024.
+constexpr int WIDE_NT = 512;
+bool wide_points(int active) { return active <= env_int("STAB_WIDE_POINTS", 256); }
+
 struct KSParams {
   int m, keep, maxcycles, ir;
   double tol;
+  bool track = false;      // fallback of a tracked point (k_schur_seq)
 };
 
 template <typename T, int NB>
@@ -605,23 +617,34 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
   const cx<T> *mats = (const cx<T> *)B.mats, *blks = (const cx<T> *)B.blks;
   int nevmax = 1;
   for (const auto &d : B.h) nevmax = std::max(nevmax, d.nev);
-  const size_t lds_schur = schur_lds_bytes(kp.m, nevmax);
+  const size_t lds_schur = kp.track ? sizeof(zd) * (2 * kp.m * kp.m + kp.m + KS_NEVMAX * kp.m) : schur_lds_bytes(kp.m, nevmax);
   std::vector<KSState> hs(npts);
   cycles_max = 0;
   ms_arnoldi = 0.0;
+  int active = npts;        // points that have not stopped
   for (int cyc = 0; cyc < kp.maxcycles; ++cyc) {
     HIPCHECK(c, hipEventRecord(c->ev[5], c->stream));
-    if (full)
-      hipLaunchKernelGGL((k_arnoldi<T, NB, 256, true>), dim3(npts), dim3(256), lds_arn, c->stream, B.pts, mats,
-                         B.pivs, blks, B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax,
-                         B.nymax, B.nvecmax, cyc == 0 ? 1 : 0);
-    else
-      hipLaunchKernelGGL((k_arnoldi<T, NB, 256, false>), dim3(npts), dim3(256), lds_arn, c->stream, B.pts, mats,
-                         B.pivs, blks, B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax,
-                         B.nymax, B.nvecmax, cyc == 0 ? 1 : 0);
+    const bool wide = kp.track || wide_points(active);
+    auto arnoldi = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(npts), dim3(wide ? WIDE_NT : 256), lds_arn, c->stream, B.pts, mats, B.pivs, blks,
+                         B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax, B.nymax, B.nvecmax,
+                         cyc == 0 ? 1 : 0);
+    };
+    if (sizeof(T) == 8 && kp.track) {
+      if constexpr (sizeof(T) == 8) {
+        if (full) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
+        else arnoldi(k_arnoldi<T, NB, WIDE_NT, false, true>);
+      }
+    } else if (full) {
+      if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
+      else arnoldi(k_arnoldi<T, NB, 256, true>);
+    } else if constexpr (sizeof(T) == 8) {        // FP32 factors come with refinement, the full operator
+      if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, false>);
+      else arnoldi(k_arnoldi<T, NB, 256, false>);
+    }
     HIPCHECK(c, hipEventRecord(c->ev[6], c->stream));
-    hipLaunchKernelGGL(k_schur, dim3(npts), dim3(128), lds_schur, c->stream, B.pts, B.small, B.state, kp.m, kp.keep,
-                       kp.tol);
+    hipLaunchKernelGGL(kp.track ? k_schur_seq : k_schur, dim3(npts), dim3(kp.track ? 64 : 128), lds_schur, c->stream, B.pts,
+                       B.small, B.state, kp.m, kp.keep, kp.tol);
     HIPCHECK(c, hipGetLastError());
     HIPCHECK(c, hipMemcpyAsync(hs.data(), B.state, sizeof(KSState) * npts, hipMemcpyDeviceToHost, c->stream));
     HIPCHECK(c, hipStreamSynchronize(c->stream));
@@ -634,14 +657,16 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
     int ndone = 0;
     for (auto &s : hs) ndone += (s.done != 0);
     if (ndone == npts || cyc == kp.maxcycles - 1) break;
-    hipLaunchKernelGGL((k_restart<256, 32>), dim3(npts), dim3(256), 0, c->stream, B.pts, B.V, B.small, B.state,
+    active = npts - ndone;
+    hipLaunchKernelGGL((k_restart<256, 32>), dim3(npts, (B.nvecmax + 255) / 256), dim3(256), 0, c->stream, B.pts, B.V, B.small, B.state,
                        kp.m, kp.keep);
     HIPCHECK(c, hipGetLastError());
   }
   nconv = 0;
   for (auto &s : hs) nconv += (s.done == 1);
-  hipLaunchKernelGGL(k_final<256>, dim3(npts), dim3(256), lds, c->stream, B.pts, B.V, B.small, B.coef, B.ops, B.norms,
-                     kp.m, B.eval, B.evec, B.resid, B.ff, B.npadmax, B.nymax, B.nvecmax);
+  const bool wide = wide_points(npts);
+  hipLaunchKernelGGL(wide ? k_final<WIDE_NT> : k_final<256>, dim3(npts), dim3(wide ? WIDE_NT : 256), lds, c->stream, B.pts, B.V,
+                     B.small, B.coef, B.ops, B.norms, kp.m, B.eval, B.evec, B.resid, B.ff, B.npadmax, B.nymax, B.nvecmax);
   HIPCHECK(c, hipGetLastError());
   return STAB_OK;
 }
@@ -1040,7 +1065,8 @@ struct RunInfo {
 
 // Validate, build the batch, assemble, factor and run Krylov-Schur + k_final;
 // results stay on the device in B.
-static int solve_run(stab_ctx *c, int npts, const stab_point *pts, int mode, Batch &B, RunInfo &ri) {
+static int solve_run(stab_ctx *c, int npts, const stab_point *pts, int mode, Batch &B, RunInfo &ri,
+                     bool track = false) {
   if (!c) return STAB_E_ARG;
   if (npts <= 0 || !pts) return fail(c, STAB_E_ARG, "npts/pts");
   if (mode != STAB_MODE_PLAIN_F64 && mode != STAB_MODE_MIXED) return fail(c, STAB_E_ARG, "unknown mode %d", mode);
@@ -1058,6 +1084,7 @@ static int solve_run(stab_ctx *c, int npts, const stab_point *pts, int mode, Bat
   kp.maxcycles = env_int("STAB_KS_CYCLES", 10);
   kp.ir = (mode == STAB_MODE_MIXED) ? -env_int("STAB_IR_MAX", 12) : 0;   // adaptive refinement
   kp.tol = 1e-12;
+  kp.track = track;
   if (kp.m > KS_MMAX || kp.keep > 32 || kp.keep < nevmax || kp.keep >= kp.m)
     return fail(c, STAB_E_ARG, "Krylov-Schur sizes m=%d keep=%d nev=%d", kp.m, kp.keep, nevmax);
   const bool f32 = (mode == STAB_MODE_MIXED);
@@ -1266,7 +1293,7 @@ static int lead_krylov(stab_ctx *c, int npts, const stab_point *pts, int mode, c
   Batch B;
   RunInfo ri;
   int rc;
-  if ((rc = solve_run(c, npts, pts, mode, B, ri)) != STAB_OK) return rc;
+  if ((rc = solve_run(c, npts, pts, mode, B, ri, nearest)) != STAB_OK) return rc;
   const size_t ne = (size_t)KS_NEVMAX * npts;
   std::vector<zd> ev(ne);
   std::vector<double> rs(ne), ff(ne);
@@ -1344,7 +1371,8 @@ static int lead_invit(stab_ctx *c, int npts, const stab_point *pts, int mode, in
   // points' first passes, instead of in a second launch whose few work-groups
   // leave the GPU idle; it needs only 2 NT more LDS entries, as it reuses the
   // first pass's vectors.  STAB_FUSE2=0 issues k_invit2 after k_invit.
-  const size_t lds_f = lds + sizeof(zd) * 2 * 256;
+  const bool wide = wide_points(npts);
+  const size_t lds_f = lds + (wide ? 0 : sizeof(zd) * 2 * 256);   // a wide work-group has tmp for two right-hand sides
   const bool fuse2 = env_int("STAB_FUSE2", 1) && lds_f <= 160 * 1024;
   const bool do2 = fuse2 || lds2 <= 160 * 1024;
   const size_t lds1 = fuse2 ? lds_f : lds;
@@ -1381,16 +1409,18 @@ static int lead_invit(stab_ctx *c, int npts, const stab_point *pts, int mode, in
     zd *ev2 = B.eval + npts;
     double *rs2 = B.resid + npts, *ff2 = B.ff + npts;    // 2 npts entries each (KS_NEVMAX npts allocated)
     const int want = nearest ? 1 : 0;
-    if (f32)
-      hipLaunchKernelGGL((k_invit<float, 16, 256>), dim3(npts), dim3(256), lds1, c->stream, B.pts, (const zf *)B.mats,
-                         B.pivs, (const zf *)B.blks, B.scales, B.coef, B.ops, B.norms, maxit, tol, B.eval, B.evec,
-                         B.resid, B.ff, B.iters, B.flag, B.npadmax, B.nymax, B.order, fuse2 ? 2 : (do2 ? 1 : 0), want,
-                         (const int *)B.info, ev2, rs2, ff2);
-    else
-      hipLaunchKernelGGL((k_invit<double, 16, 256>), dim3(npts), dim3(256), lds1, c->stream, B.pts, (const zd *)B.mats,
-                         B.pivs, (const zd *)B.blks, B.scales, B.coef, B.ops, B.norms, maxit, tol, B.eval, B.evec,
-                         B.resid, B.ff, B.iters, B.flag, B.npadmax, B.nymax, B.order, fuse2 ? 2 : (do2 ? 1 : 0), want,
-                         (const int *)B.info, ev2, rs2, ff2);
+    auto invit = [&](auto kernel, auto *mats) {
+      hipLaunchKernelGGL(kernel, dim3(npts), dim3(wide ? WIDE_NT : 256), lds1, c->stream, B.pts, mats, B.pivs,
+                         (decltype(mats))B.blks, B.scales, B.coef, B.ops, B.norms, maxit, tol, B.eval, B.evec, B.resid, B.ff,
+                         B.iters, B.flag, B.npadmax, B.nymax, B.order, fuse2 ? 2 : (do2 ? 1 : 0), want, (const int *)B.info,
+                         ev2, rs2, ff2);
+    };
+    const zf *mf = (const zf *)B.mats;
+    const zd *md = (const zd *)B.mats;
+    if (f32 && wide) invit(k_invit<float, 16, WIDE_NT>, mf);
+    else if (f32) invit(k_invit<float, 16, 256>, mf);
+    else if (wide) invit(k_invit<double, 16, WIDE_NT>, md);
+    else invit(k_invit<double, 16, 256>, md);
     HIPCHECK(c, hipGetLastError());
     if ((rc2 = mark(4)) != STAB_OK) return rc2;
     if (do2 && !fuse2) {
@@ -1410,7 +1440,7 @@ static int lead_invit(stab_ctx *c, int npts, const stab_point *pts, int mode, in
   };
   if (use_graph) {
     std::vector<long long> sig = {npts, f32, maxit, (long long)lds, B.npadmax, B.nymax, B.nvecmax,
-                                  (long long)B.nscales, (long long)lds2, do2, nearest, fuse2};
+                                  (long long)B.nscales, (long long)lds2, do2, nearest, fuse2, wide};
     for (int key : B.nys) { sig.push_back(key); sig.push_back(B.op_off[key]); }
     for (const void *q : {(const void *)B.pts, (const void *)B.prof, (const void *)B.ops, (const void *)B.coef,
                           (const void *)B.grid, (const void *)B.mats, (const void *)B.pivs, (const void *)B.blks,

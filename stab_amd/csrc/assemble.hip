@@ -25,8 +25,9 @@ __global__ __launch_bounds__(256) void k_rowscale(const PointDev *__restrict__ p
       double vyy[5];
       for (int q = 0; q < 5; ++q) form_coef(P, node, FORM_SHIFTED, p, q, P.shift, bh[q], vyy[q], dh[q]);
       mx2 = 0.0;
-      for (int j = 0; j < ny; ++j) {
-        const double d1 = D1[(size_t)j * ny + i], d2 = D2[(size_t)j * ny + i];
+      struct D12 { double d1, d2; };
+      for_loaded<8>(ny, [&](int j) { return D12{D1[(size_t)j * ny + i], D2[(size_t)j * ny + i]}; }, [&](int j, D12 d) {
+        const double d1 = d.d1, d2 = d.d2;
         for (int q = 0; q < 5; ++q) {
           zd v;
           if (kind == ROW_GENERIC || (!walle_vyy_d1(P) && q < 4)) v = bh[q] * d1 - mk(vyy[q] * d2, 0.0);
@@ -35,7 +36,7 @@ __global__ __launch_bounds__(256) void k_rowscale(const PointDev *__restrict__ p
           if (j == i) v = v + dh[q];
           mx2 = fmax(mx2, abs2(v));
         }
-      }
+      });
     }
     const double mx = sqrt(mx2);
     scales[P.scale_off + r] = (mx > 0.0) ? exp2(-rint(log2(mx))) : 1.0;
@@ -116,8 +117,9 @@ __global__ __launch_bounds__(256) void k_assemble_rows(const PointDev *__restric
 #pragma unroll
   for (int q = 0; q < 5; ++q) form_coef(P, node, FORM_SHIFTED, p, q, P.shift, bh[q], vyy[q], dh[q]);
   const double *D1 = ops + P.op_off, *D2 = D1 + (size_t)ny * ny, *dt2w = D2 + (size_t)ny * ny;
-  for (int j = 0; j < ny; ++j) {
-    const double d1 = D1[(size_t)j * ny + i], d2 = D2[(size_t)j * ny + i];
+  struct D12 { double d1, d2; };
+  for_loaded<4>(ny, [&](int j) { return D12{D1[(size_t)j * ny + i], D2[(size_t)j * ny + i]}; }, [&](int j, D12 d) {
+    const double d1 = d.d1, d2 = d.d2;
 #pragma unroll
     for (int q = 0; q < 5; ++q) {
       zd v;
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(256) void k_assemble_rows(const PointDev *__restric
       if (scaled) v = v * (rs * dc[c]);
       store_stream(M + (size_t)c * ld + r, cvt<T>(v));
     }
-  }
+  });
   for (int c = n; c < P.npad; ++c) store_stream(M + (size_t)c * ld + r, czero<T>());
 }
 

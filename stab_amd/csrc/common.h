@@ -94,6 +94,46 @@ constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;
 template <typename T> __device__ inline T quad_xor1(T x) { return dpp_move<DPP_XOR1>(x); }
 template <typename T> __device__ inline T quad_xor2(T x) { return dpp_move<DPP_XOR2>(x); }
 
+// Exchanges between the 16-lane rows of a wave (permlane16_swap, permlane32_swap):
+// x plus its value in lane ^ 16 or lane ^ 32, and the values of the four rows
+// at this lane's place in its row.
+struct rows2 { double a, b; };
+template <int W> __device__ inline rows2 row_swap(double x) {
+  const long long v = __double_as_longlong(x);
+  const unsigned lo = (unsigned)(v & 0xffffffffLL), hi = (unsigned)(v >> 32);
+  rows2 r;
+  if constexpr (W == 16) {         // a: rows 0 0 2 2, b: rows 1 1 3 3
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    r.a = __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0]));
+    r.b = __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+  } else {                         // a: rows 0 1 0 1, b: rows 2 3 2 3
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    r.a = __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0]));
+    r.b = __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+  }
+  return r;
+}
+template <int W> __device__ inline double add_rows(double x) { const rows2 r = row_swap<W>(x); return r.a + r.b; }
+// ((row 0 + row 1) + row 2) + row 3
+__device__ inline double sum_rows_in_order(double x) {
+  const rows2 p = row_swap<16>(x), e = row_swap<32>(p.a), o = row_swap<32>(p.b);
+  return ((e.a + o.a) + e.b) + o.b;
+}
+// Sum over the wave in every lane, the pairs of lane ^ 32, ^ 16, ... ^ 1 added
+// in that order (after the first three every row holds two equal halves, so
+// rotating it by 4 exchanges lane ^ 4).
+__device__ inline double wave_sum_xor(double x) {
+  x = add_rows<32>(x);
+  x = add_rows<16>(x);
+  x += dpp_move<0x128>(x);
+  x += dpp_move<0x124>(x);
+  x += quad_xor2(x);
+  x += quad_xor1(x);
+  return x;
+}
+
 // Arg-max of (v, i) over the 64 lanes of a wave: larger v, and the lower i
 // among equal v, a total order when no v is NaN, so the result does not
 // depend on the order of the reduction; returned in every lane.  Row shifts

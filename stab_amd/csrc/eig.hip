@@ -50,9 +50,14 @@ struct KSState {
 //   1. y_top <- inv(D) y_top: lane (i, q) sums columns 16q..16q+15 of row i
 //      of the column-major inverse (a wave reads 64 consecutive entries per
 //      load); the four partial sums meet in tmp (NT = 256 entries);
-//   2. the rows below (forward) or above (backward): lane (g, q) of a row
-//      group g (E rows, E = 16 bytes / entry size) loads 16 columns of
-//      quarter q and the quarters are summed by shuffles.
+//   2. the rows below (forward) or above (backward): a row group g is E rows
+//      (E = 16 bytes / entry size); the 16 lanes of a DPP row take 16
+//      consecutive groups, the four DPP rows of a wave the four quarters q of
+//      the 64 columns, and the quarters are summed across the rows.  Consecutive
+//      lanes so read consecutive 16-byte entries; with the quarters on
+//      consecutive lanes instead every group of four lanes met four cache
+//      lines, and a CU could not take in more than 13 bytes a cycle, at any
+//      number of loads in flight.
 // Columns of a partial last block (bs < 64) beyond bs are never loaded.
 // y, work in LDS (npad); tmp in LDS (NT entries).
 // ---------------------------------------------------------------------------
@@ -113,31 +118,34 @@ __device__ inline void solve_diag(const cx<T> *__restrict__ inv, int k0, int bs,
 // as soon as the entry is used, so loads stay in flight through the arithmetic
 // and the reductions; the other kernels, tighter on registers, load pass by
 // pass.  The arithmetic is the same either way.
-// Branch-free: column indexes past bs are clamped to bs - 1 (tmp is zero
-// there) and rows past r1 to the last row group (not written back).
+// Branch-free: rows past r1 take the last row group (not written back).
 template <typename T, int NT, int NR, bool PIPE = false>
 __device__ inline void solve_update(const cx<T> *__restrict__ A, int lda, int k0, int bs, int r0, int r1,
                                     zd *const (&y)[NR], const zd *tmp) {
   typedef Row16<T> R;
   typedef typename R::V V;
   constexpr int E = R::E, G = NT / 4;        // G row groups of E rows per pass
-  const int t = threadIdx.x, q = t & 3, g = t >> 2;
+  const int t = threadIdx.x, q = (t >> 4) & 3, g = (t >> 6) * 16 + (t & 15);
   const int ldv = lda / E;
-  const V *base = (const V *)A;
-  int coff[16];                              // this lane's 16 columns, in V units
-#pragma unroll
-  for (int j = 0; j < 16; ++j) coff[j] = (k0 + min(q * 16 + j, bs - 1)) * ldv;
+  // bs is 32 or 64: the upper columns of a 32-wide last block meet zeros of
+  // tmp, from columns in range.  32-bit lane offsets from uniform bases.
+  const int col = k0 + (q * 16 < bs ? q * 16 : q * 16 - 32);
+  auto offset = [&](int rb) { return (unsigned)((col * ldv + min(rb + g * E, r1 - E) / E) * (int)sizeof(V)); };
+  auto entry = [&](int j, unsigned off) {
+    return __builtin_nontemporal_load((const V *)((const char *)A + (size_t)j * ldv * sizeof(V) + off));
+  };
   V v[16];
   auto load = [&](int rb) {
-    const int rl = min(rb + g * E, r1 - E);
+    const unsigned off = offset(rb);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = __builtin_nontemporal_load(base + coff[j] + rl / E);
+    for (int j = 0; j < 16; ++j) v[j] = entry(j, off);
   };
   // one pass over rows rb .. rb + G E; with NEXT, each entry's register is
   // reloaded with the next pass's entry (rows rn ..) as soon as it is used
   auto pass = [&](int rb, int rn, auto next) {
     constexpr bool NEXT = decltype(next)::value;
-    const int row = rb + g * E, rln = min(rn + g * E, r1 - E);
+    const int row = rb + g * E;
+    const unsigned off = offset(rn);
     zd a[NR][E];
 #pragma unroll
     for (int r = 0; r < NR; ++r)
@@ -151,14 +159,14 @@ __device__ inline void solve_update(const cx<T> *__restrict__ A, int lda, int k0
 #pragma unroll
         for (int e = 0; e < E; ++e) a[r][e] = cfma(a[r][e], R::get(v[j], e), mj);
       }
-      if (NEXT) v[j] = __builtin_nontemporal_load(base + coff[j] + rln / E);
+      if (NEXT) v[j] = entry(j, off);
     }
 #pragma unroll
     for (int r = 0; r < NR; ++r)
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        a[r][e].x += quad_xor1(a[r][e].x); a[r][e].y += quad_xor1(a[r][e].y);
-        a[r][e].x += quad_xor2(a[r][e].x); a[r][e].y += quad_xor2(a[r][e].y);
+        a[r][e].x = add_rows<32>(add_rows<16>(a[r][e].x));
+        a[r][e].y = add_rows<32>(add_rows<16>(a[r][e].y));
       }
     if (row < r1 && q == 0) {
 #pragma unroll
@@ -242,33 +250,239 @@ __device__ __forceinline__ void lu_solve_n(const PointDev &P, const cx<T> *__res
   }
 }
 
+// The value of lane l (the same l in every lane).
+__device__ inline double lane_get(double x, int l) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)(unsigned int)(b & 0xffffffffLL), l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
+}
+__device__ inline zd lane_get(zd x, int l) { return mk(lane_get(x.x, l), lane_get(x.y, l)); }
+// Sum over the wave, in every lane (row shifts, then row broadcasts; lanes
+// without a source add nothing).
+template <int CTRL, int RM> __device__ inline double dpp_or_zero(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b & 0xffffffffLL), CTRL, RM, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RM, 0xF, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
+}
+__device__ inline double wave_sum(double x) {
+  x += dpp_or_zero<0x111, 0xF>(x);
+  x += dpp_or_zero<0x112, 0xF>(x);
+  x += dpp_or_zero<0x114, 0xF>(x);
+  x += dpp_or_zero<0x118, 0xF>(x);
+  x += dpp_or_zero<0x142, 0xA>(x);
+  x += dpp_or_zero<0x143, 0xC>(x);
+  return lane63(x);
+}
+
+// The same solve for work-groups of more than four waves, for batches that
+// leave CUs idle (at most a work-group per CU): what bounds it then is the
+// chain of 2 nblk block steps, not memory, so
+//   * NT / 4 row groups x 64 columns are in flight at once, and every register
+//     of a pass is reloaded, as soon as it is used, with the entry of the next
+//     pass, across block steps too: the loads of a step do not depend on the
+//     solution, so they arrive while the step before is finished;
+//   * the same holds for the entries of the diagonal-block inverse (four waves,
+//     its quarters on the DPP rows, no partial sums in LDS) and for the
+//     interchange record (one entry per thread);
+//   * a step has two barriers (four with interchanges).
+// Every sum is formed in the order of lu_solve_n, so the result is the same.
+// One point of N = 96 in FP64 (n = 480, 3.7 MB): 134 us with 256 threads,
+// 52 us with 512.  The factor comes with plain loads: at these batch sizes
+// it can stay in the caches from one solve to the next.  kb is 32 or 64: the
+// lanes of the upper columns of a 32-wide last block take in-range columns
+// and meet the zeros of tmp.
+template <typename T, int NT, int NR>
+__device__ __forceinline__ void lu_solve_wide(const PointDev &P, const cx<T> *__restrict__ A, const int *__restrict__ ipiv,
+                                              const cx<T> *__restrict__ blk, zd *const (&y)[NR], zd *tmp) {
+  typedef Row16<T> R;
+  typedef typename R::V V;
+  constexpr int BS = SOLVE_BS, E = R::E, G = NT / 4, CPL = 16;
+  static_assert(NT >= 4 * BS, "four waves for the diagonal product");
+  const int n = P.npad, lda = P.npad, t = threadIdx.x;
+  const int nblk = (n + BS - 1) / BS, q = (t >> 4) & 3, g = (t >> 6) * 16 + (t & 15), ldv = lda / E;
+  const bool dwave = __builtin_amdgcn_readfirstlane(t >> 6) < 4;     // waves of the diagonal product
+  const int dr = g & (BS - 1);                                        // its row; q its quarter of the columns
+  const int *rec0 = ipiv + 2 * n;
+  const bool progressive = rec0[0] != 0;
+  if (!progressive) {
+    const int *perm = ipiv + n;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      zd w[(1280 + NT - 1) / NT];
+#pragma unroll
+      for (int k = 0; k < (1280 + NT - 1) / NT; ++k) if (t + k * NT < n) w[k] = y[r][perm[t + k * NT]];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < (1280 + NT - 1) / NT; ++k) if (t + k * NT < n) y[r][t + k * NT] = w[k];
+      __syncthreads();
+    }
+  }
+  // first row of pass 0 and end row of step s (forward steps 0 .. nblk - 1,
+  // then backward over the blocks nblk - 1 .. 0)
+  auto rows = [&](int s, int &k0, int &r0, int &r1) {
+    const int b = s < nblk ? s : 2 * nblk - 1 - s;
+    k0 = b * BS;
+    r0 = s < nblk ? min(k0 + BS, n) : 0;
+    r1 = s < nblk ? n : k0;
+  };
+  // Byte offsets of this lane's first entry of a pass and of its first column
+  // of the step's diagonal inverse: 32-bit lane offsets from bases that are the
+  // same for the work-group, so sixteen loads need no lane addresses of their own.
+  auto entry = [&](int k0, int rb, int r1) {
+    const int qc = (k0 + q * 16 < n) ? q * 16 : q * 16 - 32;
+    return (unsigned)(((k0 + qc) * ldv + max(min(rb + g * E, r1 - E), 0) / E) * (int)sizeof(V));
+  };
+  auto load_v = [&](int j, unsigned off) { return *(const V *)((const char *)A + (size_t)j * ldv * sizeof(V) + off); };
+  const unsigned doff = (unsigned)((q * CPL * BS + dr) * (int)sizeof(cx<T>));
+  auto inv_base = [&](int s) {
+    const int b = s < nblk ? s : 2 * nblk - 1 - s;
+    return (const char *)(blk + ((size_t)(s < nblk ? 0 : nblk) + b) * BS * BS);
+  };
+  auto load_d = [&](int j, const char *c) { return *(const cx<T> *)(c + (size_t)j * BS * sizeof(cx<T>) + doff); };
+  auto records = [&](int s, int &ns, int &src, int &dst) {
+    const int *rec = rec0 + 1 + (size_t)min(s, nblk - 1) * LU_PREC;
+    ns = rec[0];
+    const int e = min(t, 2 * BS - 1);
+    dst = rec[1 + e];
+    src = rec[1 + 2 * BS + e];
+  };
+  int k0, r0, r1, ns = 0, src = 0, dst = 0;
+  rows(0, k0, r0, r1);
+  V v[16];
+  cx<T> d[CPL];
+  {
+    const unsigned p = entry(k0, r0, r1);
+    const char *c = inv_base(0);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = load_v(j, p);
+    if (dwave) {
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) d[j] = load_d(j, c);
+    }
+  }
+  if (progressive) records(0, ns, src, dst);
+#pragma unroll 1
+  for (int s = 0; s < 2 * nblk; ++s) {
+    const int bs = min(BS, n - k0);
+    if (progressive && s < nblk) {
+      if (ns > 0) {                                     // at most 2 BS <= NT entries
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          zd w = czero<double>();
+          if (t < ns) w = y[r][src];
+          __syncthreads();
+          if (t < ns) y[r][dst] = w;
+        }
+        __syncthreads();
+      }
+      records(s + 1, ns, src, dst);
+    }
+    int k0n = k0, r0n = r0, r1n = r1;
+    if (s + 1 < 2 * nblk) rows(s + 1, k0n, r0n, r1n);
+    if (dwave) {
+      const char *c = inv_base(min(s + 1, 2 * nblk - 1));
+      zd a[NR];
+#pragma unroll
+      for (int r = 0; r < NR; ++r) a[r] = czero<double>();
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) {
+        const int kk = k0 + min(q * CPL + j, bs - 1);  // entries past bs are zero
+#pragma unroll
+        for (int r = 0; r < NR; ++r) a[r] = cfma(a[r], cvt<double>(d[j]), y[r][kk]);
+        d[j] = load_d(j, c);
+      }
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        a[r] = mk(sum_rows_in_order(a[r].x), sum_rows_in_order(a[r].y));
+        // tmp, not y: other rows of the block still read y
+        if (q == 0) tmp[r * BS + dr] = (dr < bs) ? a[r] : czero<double>();
+      }
+    }
+    __syncthreads();
+    if (t < NR * BS && (t & (BS - 1)) < bs) (t < BS ? y[0] : y[NR - 1])[k0 + (t & (BS - 1))] = tmp[t];
+    static_assert(NR <= 2, "one or two right-hand sides");
+#pragma unroll 1
+    for (int rb = r0; rb < r1; rb += G * E) {
+      const bool last = rb + G * E >= r1;
+      const unsigned p = last ? entry(k0n, r0n, r1n) : entry(k0, rb + G * E, r1);
+      zd a[NR][E];
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int e = 0; e < E; ++e) a[r][e] = czero<double>();
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+          const zd mj = tmp[r * BS + q * 16 + j];
+#pragma unroll
+          for (int e = 0; e < E; ++e) a[r][e] = cfma(a[r][e], R::get(v[j], e), mj);
+        }
+        v[j] = load_v(j, p);
+      }
+      const int row = rb + g * E;
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+          a[r][e].x = add_rows<32>(add_rows<16>(a[r][e].x));
+          a[r][e].y = add_rows<32>(add_rows<16>(a[r][e].y));
+        }
+      if (row < r1 && q == 0) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+#pragma unroll
+          for (int e = 0; e < E; ++e) y[r][row + e] = y[r][row + e] - a[r][e];
+      }
+    }
+    if (r0 >= r1) {                                     // nothing to update: fetch the next step's first pass
+      const unsigned p = entry(k0n, r0n, r1n);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = load_v(j, p);
+    }
+    __syncthreads();
+    k0 = k0n; r0 = r0n; r1 = r1n;
+  }
+}
+
+template <typename T, int NT, int NR, bool PIPE = false>
+__device__ __forceinline__ void lu_solve_many(const PointDev &P, const cx<T> *__restrict__ A, const int *__restrict__ ipiv,
+                                              const cx<T> *__restrict__ blk, zd *const (&y)[NR], zd *tmp, zd *work) {
+  if constexpr (NT > 256) lu_solve_wide<T, NT, NR>(P, A, ipiv, blk, y, tmp);
+  else lu_solve_n<T, NT, NR, PIPE>(P, A, ipiv, blk, y, tmp, work);
+}
+
 template <typename T, int NT, bool PIPE = false>
 __device__ __forceinline__ void lu_solve(const PointDev &P, const cx<T> *__restrict__ A, const int *__restrict__ ipiv,
                                          const cx<T> *__restrict__ blk, zd *y, zd *tmp, zd *work) {
   zd *const ys[1] = {y};
-  lu_solve_n<T, NT, 1, PIPE>(P, A, ipiv, blk, ys, tmp, work);
+  lu_solve_many<T, NT, 1, PIPE>(P, A, ipiv, blk, ys, tmp, work);
 }
 
 // Block-wide reduction of NV complex partial sums; result broadcast to all.
+// Partial sums come from the first RT = 256 threads (red_first, RT), so
+// the result does not depend on the size of the work-group.
+__device__ inline int red_first() { return threadIdx.x < 256 ? (int)threadIdx.x : 1 << 30; }
+constexpr int RT = 256;
 template <int NT, int NV>
 __device__ void block_reduce(zd (&v)[NV], zd *red) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  if (NT <= RT || w < RT / 64) {
 #pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    for (int off = 32; off > 0; off >>= 1) {
-      v[k].x += __shfl_xor(v[k].x, off);
-      v[k].y += __shfl_xor(v[k].y, off);
+    for (int k = 0; k < NV; ++k) v[k] = mk(wave_sum_xor(v[k].x), wave_sum_xor(v[k].y));
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) red[w * NV + k] = v[k];
     }
-  }
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) red[w * NV + k] = v[k];
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     zd s = czero<double>();
-    for (int ww = 0; ww < NT / 64; ++ww) s = s + red[ww * NV + k];
+#pragma unroll
+    for (int ww = 0; ww < RT / 64; ++ww) s = s + red[ww * NV + k];
     v[k] = s;
   }
   __syncthreads();
@@ -277,9 +491,26 @@ __device__ void block_reduce(zd (&v)[NV], zd *red) {
 template <int NT>
 __device__ double block_norm2(const zd *x, int len, zd *red) {
   zd v[1] = {czero<double>()};
-  for (int r = threadIdx.x; r < len; r += NT) v[0].x += abs2(x[r]);
+  for (int r = red_first(); r < len; r += RT) v[0].x += abs2(x[r]);
   block_reduce<NT, 1>(v, red);
   return v[0].x;
+}
+
+// First index of largest value over the work-group: (v, i) per thread, v = -1
+// where it has none (a NaN never becomes a candidate); red: NT / 64 entries.
+template <int NT>
+__device__ int block_argmax(double v, int i, zd *red) {
+  const int t = threadIdx.x;
+  wave_argmax(v, i);
+  if ((t & 63) == 0) red[t >> 6] = mk(v, (double)i);
+  __syncthreads();
+#pragma unroll 4
+  for (int w = 0; w < NT / 64; ++w) {
+    const zd c = red[w];
+    if (c.x > v || (c.x == v && (int)c.y < i)) { v = c.x; i = (int)c.y; }
+  }
+  __syncthreads();
+  return i;
 }
 
 // Shared-memory layout of the operator kernels (dynamic LDS, zd units).
@@ -290,10 +521,12 @@ struct OpLds {
   zd *y, *rhs, *res, *X1, *X2, *z, *red, *tmp, *w2;
   // nvecmax: longest Krylov vector (2 n for spatial points).  w2, the gather
   // buffer of the solves, aliases X1/X2 (10 ny >= npad), which are idle then.
-  __device__ OpLds(zd *base, const PointDev &P, int npadmax, int nymax, int full, int nvecmax) {
+  // red: NT / 64 sums of up to 8 values; tmp: NT entries (256 threads) or 64
+  // per right-hand side.
+  __device__ OpLds(zd *base, int nt, int npadmax, int nymax, int full, int nvecmax) {
     red = base;
-    tmp = red + 64;
-    y = tmp + 256;
+    tmp = red + (nt > 256 ? 128 : 64);
+    y = base + 320;
     z = y + npadmax;
     if (full) {
       rhs = z + nvecmax;
@@ -338,7 +571,7 @@ __device__ bool shifted_solve(const PointDev &P, const cx<T> *A, const int *ipiv
     __syncthreads();
     lu_solve<T, NT, PIPE>(P, A, ipiv, Lb, L.res, L.tmp, L.w2);
     zd nrm[2] = {czero<double>(), czero<double>()};
-    for (int r = t; r < n; r += NT) {
+    for (int r = red_first(); r < n; r += RT) {
       const zd d = L.res[r] * dc[r];
       L.y[r] = L.y[r] + d;
       nrm[0].x += abs2(d);
@@ -427,8 +660,8 @@ __device__ inline unsigned point_seed(const PointDev &P) {
 // ---------------------------------------------------------------------------
 // Arnoldi expansion from column j0 to m (CGS2).  V column-major, ld = ldv.
 // ---------------------------------------------------------------------------
-template <typename T, int NB, int NT, bool FULL>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 3))) void k_arnoldi(const PointDev *__restrict__ pts, const cx<T> *__restrict__ mats,
+template <typename T, int NB, int NT, bool FULL, bool GS4 = false>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FULL || NT > 256 ? 2 : 3))) void k_arnoldi(const PointDev *__restrict__ pts, const cx<T> *__restrict__ mats,
                                                 const int *__restrict__ pivs, const cx<T> *__restrict__ blks,
                                                 const double *__restrict__ scales, const zd *__restrict__ coef,
                                                 const double *__restrict__ ops, zd *__restrict__ Vall,
@@ -438,7 +671,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 3
   const PointDev &P = pts[blockIdx.x];
   if (st[blockIdx.x].done) return;
   int j0 = st[blockIdx.x].j0;
-  OpLds L(lds, P, npadmax, nymax, FULL ? 1 : 0, nvecmax);
+  OpLds L(lds, NT, npadmax, nymax, FULL ? 1 : 0, nvecmax);
   const int t = threadIdx.x, nv = P.nvec;
   const size_t ldv = (size_t)nv;
   zd *V = Vall + P.vec_off;
@@ -465,34 +698,61 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : 3
   }
   for (int j = j0; j < m; ++j) {
     allok &= apply_op<T, NB, NT, FULL>(P, A, ipiv, Lb, Ub, dr, dc, coef, ops, ir, V + (size_t)j * ldv, L);
-    // two passes of classical Gram-Schmidt against V[:, 0..j]
-    for (int pass = 0; pass < 2; ++pass) {
-      for (int l0 = 0; l0 <= j; l0 += 4) {
-        zd h[4];
+    // two passes of classical Gram-Schmidt against V[:, 0..j], all
+    // coefficients of a pass at once: a wave per column forms h_l, then a
+    // thread per row subtracts the whole combination (two barriers a pass;
+    // groups of four columns with a block reduction each took 37 us a step at
+    // n = 480, 14 us here)
+    if constexpr (GS4) {
+      for (int pass = 0; pass < 2; ++pass) {
+        for (int l0 = 0; l0 <= j; l0 += 4) {
+          zd h[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) h[k] = czero<double>();
-        for (int r = t; r < nv; r += NT) {
-          const zd w = L.z[r];
+          for (int k = 0; k < 4; ++k) h[k] = czero<double>();
+          for (int r = red_first(); r < nv; r += RT) {
+            const zd w = L.z[r];
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (l0 + k <= j) h[k] = cfmac(h[k], V[(size_t)(l0 + k) * ldv + r], w);
+            for (int k = 0; k < 4; ++k)
+              if (l0 + k <= j) h[k] = cfmac(h[k], V[(size_t)(l0 + k) * ldv + r], w);
+          }
+          block_reduce<NT, 4>(h, L.red);
+          for (int r = t; r < nv; r += NT) {
+            zd w = L.z[r];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (l0 + k <= j) w = cfms(w, V[(size_t)(l0 + k) * ldv + r], h[k]);
+            L.z[r] = w;
+          }
+          if (t < 4 && l0 + t <= j) {
+            zd hv = h[0];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) if (k == t) hv = h[k];
+            H[(size_t)j * ldh + l0 + t] = H[(size_t)j * ldh + l0 + t] + hv;
+          }
+          __syncthreads();
         }
-        block_reduce<NT, 4>(h, L.red);
-        for (int r = t; r < nv; r += NT) {
-          zd w = L.z[r];
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (l0 + k <= j) w = cfms(w, V[(size_t)(l0 + k) * ldv + r], h[k]);
-          L.z[r] = w;
-        }
-        if (t < 4 && l0 + t <= j) {
-          zd hv = h[0];
-#pragma unroll
-          for (int k = 0; k < 4; ++k) if (k == t) hv = h[k];
-          H[(size_t)j * ldh + l0 + t] = H[(size_t)j * ldh + l0 + t] + hv;
-        }
-        __syncthreads();
       }
+    } else
+    for (int pass = 0; pass < 2; ++pass) {
+      for (int l = t >> 6; l <= j; l += NT / 64) {
+        const zd *Vl = V + (size_t)l * ldv + (t & 63), *z = L.z + (t & 63);
+        zd s = czero<double>();
+        for_loaded<8>((nv - (t & 63) + 63) / 64, [&](int r) { return Vl[64 * r]; },
+                      [&](int r, zd v) { s = cfmac(s, v, z[64 * r]); });
+        s = mk(wave_sum(s.x), wave_sum(s.y));
+        if ((t & 63) == 0) {
+          L.tmp[l] = s;
+          H[(size_t)j * ldh + l] = H[(size_t)j * ldh + l] + s;
+        }
+      }
+      __syncthreads();
+      for (int r = t; r < nv; r += NT) {
+        zd w = L.z[r];
+        for_loaded<8>(j + 1, [&](int l) { return V[(size_t)l * ldv + r]; },
+                      [&](int l, zd v) { w = cfms(w, v, L.tmp[l]); });
+        L.z[r] = w;
+      }
+      __syncthreads();
     }
     double nrm = sqrt(block_norm2<NT>(L.z, nv, L.red));
     if (!(nrm > 1e-300)) nrm = 1e-300;
@@ -536,31 +796,6 @@ __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__device__ inline double lane_get(double x, int l) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)(unsigned int)(b & 0xffffffffLL), l);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
-}
-__device__ inline zd lane_get(zd x, int l) { return mk(lane_get(x.x, l), lane_get(x.y, l)); }
-// Sum over the wave, in every lane (row shifts, then row broadcasts; lanes
-// without a source add nothing).
-template <int CTRL, int RM> __device__ inline double dpp_or_zero(double x) {
-  const long long b = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b & 0xffffffffLL), CTRL, RM, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, RM, 0xF, false);
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo));
-}
-__device__ inline double wave_sum(double x) {
-  x += dpp_or_zero<0x111, 0xF>(x);
-  x += dpp_or_zero<0x112, 0xF>(x);
-  x += dpp_or_zero<0x114, 0xF>(x);
-  x += dpp_or_zero<0x118, 0xF>(x);
-  x += dpp_or_zero<0x142, 0xA>(x);
-  x += dpp_or_zero<0x143, 0xC>(x);
-  return lane63(x);
-}
-
 // Rotation with c x + s y = r, c y - conj(s) x = 0, c real, the same (x, y) in
 // every lane.  Squares that would under- or overflow, and x = 0, take the
 // scaled form.
@@ -916,14 +1151,265 @@ __global__ __launch_bounds__(128) void k_schur(const PointDev *__restrict__ pts,
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same on one wave, rotation by rotation in LDS, for mode tracking only
+// (Gram-Schmidt by groups of four columns, GS4 of k_arnoldi, goes with it).
+// Tracking feeds the eigenvalue of one step into the shift of the next, and a
+// point whose residual floor lies at the acceptance limit of the inverse
+// iteration (1e-14) changes its info code with the last bits of that shift:
+// with the sums of k_schur in the fallback, 1 of 25 tracked batches returned
+// other codes.  So the fallback of a tracked point keeps this order of
+// operations; it is rare (a quarter of 16-curve batches have such a point).
+// ---------------------------------------------------------------------------
+__device__ inline void givens_seq(zd x, zd y, double &c, zd &s) {
+  const double ax = cabs(x), ay = cabs(y);
+  if (ay == 0.0) { c = 1.0; s = czero<double>(); return; }
+  if (ax == 0.0) { c = 0.0; s = conj(y) * (1.0 / ay); return; }
+  const double r = hypot(ax, ay);
+  c = ax / r;
+  s = (x * (1.0 / ax)) * conj(y) * (1.0 / r);
+}
+
+__global__ __launch_bounds__(64) void k_schur_seq(const PointDev *__restrict__ pts, zd *__restrict__ small,
+                                              KSState *__restrict__ st, int m, int keep, double tol) {
+  extern __shared__ zd sl[];
+  const PointDev &P = pts[blockIdx.x];
+  KSState S = st[blockIdx.x];
+  if (S.done) return;
+  zd *Hs = sl, *Q = Hs + m * m, *v = Q + m * m, *zz = v + m;   // zz: KS_NEVMAX * m
+  zd *Hg = small + P.small_off + SM_H;
+  zd *Qg = small + P.small_off + SM_Q;
+  zd *Yg = small + P.small_off + SM_Y;
+  zd *THg = small + P.small_off + SM_TH;
+  const int ldh = KS_MMAX + 1, t = threadIdx.x;
+  const int nev = P.nev;
+  for (int e = t; e < m * m; e += 64) {
+    const int i = e % m, j = e / m;
+    Hs[i * m + j] = Hg[(size_t)j * ldh + i];   // row-major in LDS
+    Q[i * m + j] = (i == j) ? mk(1.0, 0.0) : czero<double>();
+  }
+  const zd hlast = Hg[(size_t)(m - 1) * ldh + m];
+  __syncthreads();
+  // --- Householder reduction to Hessenberg form
+  for (int k = 0; k < m - 2; ++k) {
+    const int len = m - k - 1;
+    double nx = 0.0;
+    for (int i = 0; i < len; ++i) nx += abs2(Hs[(k + 1 + i) * m + k]);
+    double below = nx - abs2(Hs[(k + 1) * m + k]);
+    if (below <= 1e-300 * (nx + 1e-300)) continue;     // already reduced
+    nx = sqrt(nx);
+    const zd x0 = Hs[(k + 1) * m + k];
+    const double ax0 = cabs(x0);
+    const zd ph = (ax0 > 0.0) ? x0 * (1.0 / ax0) : mk(1.0, 0.0);
+    const zd alpha = ph * (-nx);
+    // v = x - alpha e1, normalised
+    for (int i = t; i < len; i += 64) v[i] = (i == 0) ? x0 - alpha : Hs[(k + 1 + i) * m + k];
+    __syncthreads();
+    double vn = 0.0;
+    for (int i = 0; i < len; ++i) vn += abs2(v[i]);
+    vn = sqrt(vn);
+    __syncthreads();
+    for (int i = t; i < len; i += 64) v[i] = v[i] * (1.0 / vn);
+    __syncthreads();
+    // H <- (I - 2 v v^H) H  on rows k+1.., columns k..m-1
+    for (int c = k + t; c < m; c += 64) {
+      zd s = czero<double>();
+      for (int i = 0; i < len; ++i) s = cfmac(s, v[i], Hs[(k + 1 + i) * m + c]);
+      for (int i = 0; i < len; ++i) Hs[(k + 1 + i) * m + c] = cfms(Hs[(k + 1 + i) * m + c], v[i], s * 2.0);
+    }
+    __syncthreads();
+    // H <- H (I - 2 v v^H) on columns k+1.., all rows; Q likewise
+    for (int rr = t; rr < 2 * m; rr += 64) {
+      zd *row = (rr < m) ? &Hs[rr * m] : &Q[(rr - m) * m];
+      zd s = czero<double>();
+      for (int i = 0; i < len; ++i) s = cfma(s, row[k + 1 + i], v[i]);
+      for (int i = 0; i < len; ++i) row[k + 1 + i] = cfms(row[k + 1 + i], s * 2.0, conj(v[i]));
+    }
+    __syncthreads();
+    if (t == 0)
+      for (int i = 2; i < len + 1; ++i) Hs[(k + i) * m + k] = czero<double>();
+    __syncthreads();
+  }
+  // --- complex QR iterations to Schur form (full T and Q)
+  const double eps = 2.220446049250313e-16;
+  int hi = m - 1, iter = 0, total = 0;
+  while (hi > 0 && total < 60 * m) {
+    int lo = hi;
+    while (lo > 0) {
+      const double sub = cabs1(Hs[lo * m + lo - 1]);
+      const double dia = cabs1(Hs[lo * m + lo]) + cabs1(Hs[(lo - 1) * m + lo - 1]);
+      if (sub <= eps * dia || sub < 1e-300) break;
+      --lo;
+    }
+    if (lo > 0) {
+      __syncthreads();
+      if (t == 0) Hs[lo * m + lo - 1] = czero<double>();
+      __syncthreads();
+    }
+    if (lo == hi) { --hi; iter = 0; continue; }
+    ++iter; ++total;
+    zd mu;
+    const zd a = Hs[(hi - 1) * m + hi - 1], b = Hs[(hi - 1) * m + hi], c = Hs[hi * m + hi - 1], d = Hs[hi * m + hi];
+    if (iter % 11 == 10) {
+      mu = d + mk(0.75 * cabs(c), 0.0);
+    } else {
+      const zd half = (a - d) * 0.5;
+      zd disc = half * half + b * c;
+      // complex sqrt
+      const double r = cabs(disc);
+      double sr = sqrt(0.5 * (r + fabs(disc.x)));
+      zd sq;
+      if (sr == 0.0) sq = czero<double>();
+      else if (disc.x >= 0) sq = mk(sr, disc.y / (2.0 * sr));
+      else sq = mk(fabs(disc.y) / (2.0 * sr), disc.y >= 0 ? sr : -sr);
+      const zd m1 = (a + d) * 0.5 + sq, m2 = (a + d) * 0.5 - sq;
+      mu = (cabs(m1 - d) < cabs(m2 - d)) ? m1 : m2;
+    }
+    for (int k = lo; k < hi; ++k) {
+      zd x, y;
+      if (k == lo) { x = Hs[lo * m + lo] - mu; y = Hs[(lo + 1) * m + lo]; }
+      else { x = Hs[k * m + k - 1]; y = Hs[(k + 1) * m + k - 1]; }
+      double cg; zd sg;
+      givens_seq(x, y, cg, sg);
+      __syncthreads();
+      const int c0 = (k > lo) ? k - 1 : lo;
+      for (int jj = c0 + t; jj < m; jj += 64) {
+        const zd p = Hs[k * m + jj], q = Hs[(k + 1) * m + jj];
+        Hs[k * m + jj] = p * cg + sg * q;
+        Hs[(k + 1) * m + jj] = q * cg - conj(sg) * p;
+      }
+      __syncthreads();
+      const int rmax = min(k + 2, hi);
+      for (int ii = t; ii <= rmax; ii += 64) {
+        const zd p = Hs[ii * m + k], q = Hs[ii * m + k + 1];
+        Hs[ii * m + k] = p * cg + conj(sg) * q;
+        Hs[ii * m + k + 1] = q * cg - sg * p;
+      }
+      for (int ii = t; ii < m; ii += 64) {
+        const zd p = Q[ii * m + k], q = Q[ii * m + k + 1];
+        Q[ii * m + k] = p * cg + conj(sg) * q;
+        Q[ii * m + k + 1] = q * cg - sg * p;
+      }
+      __syncthreads();
+      if (k > lo && t == 0) Hs[(k + 1) * m + k - 1] = czero<double>();
+      __syncthreads();
+    }
+  }
+  __syncthreads();
+  // --- reorder: bring the `keep` eigenvalues of largest modulus to the front
+  for (int pos = 0; pos < keep; ++pos) {
+    int best = pos;
+    double bv = cabs(Hs[pos * m + pos]);
+    for (int i = pos + 1; i < m; ++i) {
+      const double vv = cabs(Hs[i * m + i]);
+      if (vv > bv) { bv = vv; best = i; }
+    }
+    for (int k = best - 1; k >= pos; --k) {
+      const zd t11 = Hs[k * m + k], t22 = Hs[(k + 1) * m + k + 1];
+      double cg; zd sg;
+      givens_seq(Hs[k * m + k + 1], t22 - t11, cg, sg);
+      __syncthreads();
+      for (int jj = k + t; jj < m; jj += 64) {
+        const zd p = Hs[k * m + jj], q = Hs[(k + 1) * m + jj];
+        Hs[k * m + jj] = p * cg + sg * q;
+        Hs[(k + 1) * m + jj] = q * cg - conj(sg) * p;
+      }
+      __syncthreads();
+      for (int ii = t; ii <= k + 1; ii += 64) {
+        const zd p = Hs[ii * m + k], q = Hs[ii * m + k + 1];
+        Hs[ii * m + k] = p * cg + conj(sg) * q;
+        Hs[ii * m + k + 1] = q * cg - sg * p;
+      }
+      for (int ii = t; ii < m; ii += 64) {
+        const zd p = Q[ii * m + k], q = Q[ii * m + k + 1];
+        Q[ii * m + k] = p * cg + conj(sg) * q;
+        Q[ii * m + k + 1] = q * cg - sg * p;
+      }
+      __syncthreads();
+      if (t == 0) {
+        Hs[k * m + k] = t22;
+        Hs[(k + 1) * m + k + 1] = t11;
+        Hs[(k + 1) * m + k] = czero<double>();
+      }
+      __syncthreads();
+    }
+  }
+  // --- eigenvectors of T for the first nev (lane i handles pair i)
+  if (t < nev) {
+    const int i = t;
+    zd *z = zz + i * m;
+    const zd ti = Hs[i * m + i];
+    const double smin = fmax(eps * cabs(ti), 1e-300);
+    for (int l = 0; l < m; ++l) z[l] = czero<double>();
+    z[i] = mk(1.0, 0.0);
+    for (int l = i - 1; l >= 0; --l) {
+      zd s = czero<double>();
+      for (int c = l + 1; c <= i; ++c) s = cfma(s, Hs[l * m + c], z[c]);
+      zd d = Hs[l * m + l] - ti;
+      if (cabs(d) < smin) d = mk(smin, 0.0);
+      z[l] = czero<double>() - cdiv(s, d);
+    }
+  }
+  __syncthreads();
+  // y_i = Q z_i, normalised; residual estimate |h_{m,m-1}| |y_i[m-1]|
+  __shared__ double s_est[KS_NEVMAX];
+  if (t < nev) {
+    const int i = t;
+    const zd *z = zz + i * m;
+    double nn = 0.0;
+    zd ylast = czero<double>();
+    for (int r = 0; r < m; ++r) {
+      zd s = czero<double>();
+      for (int c = 0; c <= i; ++c) s = cfma(s, Q[r * m + c], z[c]);
+      nn += abs2(s);
+      if (r == m - 1) ylast = s;
+    }
+    const double inv = 1.0 / sqrt(nn);
+    for (int r = 0; r < m; ++r) {
+      zd s = czero<double>();
+      for (int c = 0; c <= i; ++c) s = cfma(s, Q[r * m + c], z[c]);
+      Yg[(size_t)i * KS_MMAX + r] = s * inv;
+    }
+    const zd th = Hs[i * m + i];
+    s_est[i] = cabs(hlast) * cabs(ylast) * inv / fmax(cabs(th), 1e-300);
+  }
+  __syncthreads();
+  // write T (row-major -> column-major global H) and Q, theta
+  for (int e = t; e < m * m; e += 64) {
+    const int i = e % m, j = e / m;
+    Qg[(size_t)j * KS_MMAX + i] = Q[i * m + j];
+  }
+  for (int i = t; i < m; i += 64) THg[i] = Hs[i * m + i];
+  for (int e = t; e < keep * keep; e += 64) {
+    const int i = e % keep, j = e / keep;
+    Hg[(size_t)j * ldh + i] = (i <= j) ? Hs[i * m + j] : czero<double>();
+  }
+  __syncthreads();
+  if (t == 0) {
+    double mx = 0.0;
+    for (int i = 0; i < nev; ++i) mx = fmax(mx, s_est[i]);
+    S.resmax = mx;
+    S.cycles += 1;
+    if (S.cycles == 1 || mx < 0.1 * S.best) { S.best = fmin(mx, S.cycles == 1 ? mx : S.best); S.stall = 0; }
+    else S.stall += 1;
+    S.best = fmin(S.best, mx);
+    // converged, or no tenfold progress in three cycles (an ill-conditioned
+    // cluster among the wanted pairs): stop this point
+    S.done = (mx <= tol) ? 1 : ((S.stall >= 3) ? 2 : 0);
+    st[blockIdx.x] = S;
+  }
+}
+
 // Krylov-Schur truncation to `keep` columns: V <- V Q(:, 0:keep), v_keep <- v_m,
 // H <- [T_keep; b^H], b^H = h_{m,m-1} Q(m-1, 0:keep).
 template <int NT, int KMAX>
 __global__ __launch_bounds__(NT) void k_restart(const PointDev *__restrict__ pts, zd *__restrict__ Vall,
                                                 zd *__restrict__ small, KSState *__restrict__ st, int m, int keep) {
+  // grid: x = points, y = chunks of NT rows; the first chunk's work-group also
+  // rebuilds H (the others read only V and Q)
   const PointDev &P = pts[blockIdx.x];
   KSState S = st[blockIdx.x];
-  if (S.done) return;
+  if (S.done || (int)blockIdx.y * NT >= P.nvec) return;
   __shared__ zd s_q[KS_MMAX * KMAX];
   const int t = threadIdx.x, nv = P.nvec;
   const size_t ldv = (size_t)nv;
@@ -937,22 +1423,22 @@ __global__ __launch_bounds__(NT) void k_restart(const PointDev *__restrict__ pts
   }
   const zd hlast = H[(size_t)(m - 1) * ldh + m];
   __syncthreads();
-  for (int r = t; r < nv; r += NT) {
+  if (const int r = blockIdx.y * NT + t; r < nv) {
     zd acc[KMAX];
 #pragma unroll
     for (int c = 0; c < KMAX; ++c) acc[c] = czero<double>();
-    for (int l = 0; l < m; ++l) {
-      const zd v = V[(size_t)l * ldv + r];
+    for_loaded<4>(m, [&](int l) { return V[(size_t)l * ldv + r]; }, [&](int l, zd v) {
 #pragma unroll
       for (int c = 0; c < KMAX; ++c)
         if (c < keep) acc[c] = cfma(acc[c], v, s_q[l * KMAX + c]);
-    }
+    });
     const zd vm = V[(size_t)m * ldv + r];
 #pragma unroll
     for (int c = 0; c < KMAX; ++c)
       if (c < keep) V[(size_t)c * ldv + r] = acc[c];
     V[(size_t)keep * ldv + r] = vm;
   }
+  if (blockIdx.y) return;
   __syncthreads();
   // rebuild H: T block already written by k_schur in rows/cols < keep
   for (int e = t; e < ldh * KS_MMAX; e += NT) {
@@ -1013,36 +1499,28 @@ __global__ __launch_bounds__(NT) void k_final(const PointDev *__restrict__ pts, 
                                               int nymax, int nvecmax) {
   extern __shared__ zd lds[];
   const PointDev &P = pts[blockIdx.x];
-  OpLds L(lds, P, npadmax, nymax, 1, nvecmax);
+  OpLds L(lds, NT, npadmax, nymax, 1, nvecmax);
   const int t = threadIdx.x, nv = P.nvec, n = P.n;
   const size_t ldv = (size_t)nv;
   const zd *V = Vall + P.vec_off;
   const zd *Yg = small + P.small_off + SM_Y;
   const zd *THg = small + P.small_off + SM_TH;
   zd *out = evec + P.out_off;
-  __shared__ double s_mx[NT];
-  __shared__ int s_ix[NT];
   for (int i = 0; i < P.nev; ++i) {
     const zd th = THg[i];
     const zd om = P.shift + cdiv(mk(1.0, 0.0), th);
     for (int r = t; r < nv; r += NT) {
       zd s = czero<double>();
-      for (int l = 0; l < m; ++l) s = cfma(s, V[(size_t)l * ldv + r], Yg[(size_t)i * KS_MMAX + l]);
+      for_loaded<8>(m, [&](int l) { return V[(size_t)l * ldv + r]; },
+                    [&](int l, zd v) { s = cfma(s, v, Yg[(size_t)i * KS_MMAX + l]); });
       L.z[r] = s;
     }
     __syncthreads();
     // first entry of largest modulus among the first n components
     double bm = -1.0; int bi = 0x7fffffff;
     for (int r = t; r < n; r += NT) { const double a = cabs(L.z[r]); if (a > bm) { bm = a; bi = r; } }
-    s_mx[t] = bm; s_ix[t] = bi;
-    __syncthreads();
-    if (t == 0) {
-      for (int k = 1; k < NT; ++k)
-        if (s_mx[k] > bm || (s_mx[k] == bm && s_ix[k] < bi)) { bm = s_mx[k]; bi = s_ix[k]; }
-      s_ix[0] = clamp_index(bi, n);   // all-NaN vector: no entry compares greater
-    }
-    __syncthreads();
-    const zd scale = L.z[s_ix[0]];
+    // all-NaN vector: no entry compares greater
+    const zd scale = L.z[clamp_index(block_argmax<NT>(bm, bi, L.red), n)];
     __syncthreads();
     if (scale_ok(scale))
       for (int r = t; r < nv; r += NT) L.z[r] = cdiv(L.z[r], scale);
@@ -1062,14 +1540,14 @@ __global__ __launch_bounds__(NT) void k_final(const PointDev *__restrict__ pts, 
       pencil_apply<NT>(P, coef, ops, FORM_AM, P.shift, L.z, L.y, L.X1, L.X2, L.red);
       pencil_apply<NT>(P, coef, ops, FORM_BM, P.shift, L.z, L.rhs, L.X1, L.X2, L.red);
       zd d3[3] = {czero<double>(), czero<double>(), czero<double>()};
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         d3[0] = cfmac(d3[0], L.z[r], L.y[r]);
         d3[1] = cfmac(d3[1], L.z[r], L.rhs[r]);
       }
       block_reduce<NT, 3>(d3, L.red);
       const zd om_rq = (cabs(d3[1]) > 0.0) ? cdiv(d3[0], d3[1]) : om;
       zd part[3] = {czero<double>(), czero<double>(), czero<double>()};
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         part[0].x += abs2(L.y[r] - om * L.rhs[r]);
         part[1].x += abs2(L.y[r] - om_rq * L.rhs[r]);
         part[2].x += abs2(L.z[r]);
@@ -1086,7 +1564,7 @@ __global__ __launch_bounds__(NT) void k_final(const PointDev *__restrict__ pts, 
       pencil_apply<NT>(P, coef, ops, FORM_C1, P.shift, L.z, L.rhs, L.X1, L.X2, L.red);
       pencil_apply<NT>(P, coef, ops, FORM_C2, P.shift, L.z, L.res, L.X1, L.X2, L.red);
       zd d3[3] = {czero<double>(), czero<double>(), czero<double>()};
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         d3[0] = cfmac(d3[0], L.z[r], L.y[r]);
         d3[1] = cfmac(d3[1], L.z[r], L.rhs[r]);
         d3[2] = cfmac(d3[2], L.z[r], L.res[r]);
@@ -1109,7 +1587,7 @@ __global__ __launch_bounds__(NT) void k_final(const PointDev *__restrict__ pts, 
         om_rq = czero<double>() - cdiv(d3[0], d3[1]);
       }
       zd part[3] = {czero<double>(), czero<double>(), czero<double>()};
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         part[0].x += abs2(L.y[r] + om * L.rhs[r] + (om * om) * L.res[r]);
         part[1].x += abs2(L.y[r] + om_rq * L.rhs[r] + (om_rq * om_rq) * L.res[r]);
         part[2].x += abs2(L.z[r]);
@@ -1141,7 +1619,7 @@ __global__ __launch_bounds__(NT) void k_solve_one(const PointDev *__restrict__ p
                                                   zd *__restrict__ x, int ir, int npadmax, int nymax) {
   extern __shared__ zd lds[];
   const PointDev &P = pts[blockIdx.x];
-  OpLds L(lds, P, npadmax, nymax, 1, npadmax);
+  OpLds L(lds, NT, npadmax, nymax, 1, npadmax);
   const cx<T> *A = mats + P.mat_off;
   const int *ipiv = pivs + P.piv_off;
   const cx<T> *Lb = blks + P.blk_off, *Ub = nullptr;
@@ -1232,8 +1710,7 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
                                              int maxit, double tol, int want, zd *__restrict__ eval2,
                                              zd *__restrict__ evec, double *__restrict__ resid2,
                                              double *__restrict__ ff2, int *__restrict__ iters, OpLds &L, zd *x1,
-                                             zd *x2, zd *a1, zd *b1, zd *a2, zd *b2, zd *tmp2, double *s_mx,
-                                             int *s_ix) {
+                                             zd *x2, zd *a1, zd *b1, zd *a2, zd *b2, zd *tmp2) {
   const int t = threadIdx.x, n = P.n, nv = P.nvec;
   const cx<T> *A = mats + P.mat_off;
   const int *ipiv = pivs + P.piv_off;
@@ -1256,7 +1733,7 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
       const double n1 = sqrt(block_norm2<NT>(x1, n, L.red));
       const double i1 = (n1 > 0.0) ? 1.0 / n1 : 1.0;
       zd d[1] = {czero<double>()};
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         x1[r] = x1[r] * i1;
         d[0] = cfmac(d[0], x1[r], x2[r]);
       }
@@ -1276,7 +1753,7 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
     zd pr[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) pr[k] = czero<double>();
-    for (int r = t; r < n; r += NT) {
+    for (int r = red_first(); r < n; r += RT) {
       const zd u = x1[r], v = x2[r];
       pr[0] = cfmac(pr[0], u, a1[r]); pr[1] = cfmac(pr[1], u, a2[r]);
       pr[2] = cfmac(pr[2], v, a1[r]); pr[3] = cfmac(pr[3], v, a2[r]);
@@ -1317,7 +1794,7 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
     }
     // Ritz vectors into x1, x2 and residuals into a1, a2 (element-wise in place)
     zd nr[4] = {czero<double>(), czero<double>(), czero<double>(), czero<double>()};
-    for (int r = t; r < n; r += NT) {
+    for (int r = red_first(); r < n; r += RT) {
       const zd u = x1[r], v = x2[r];
       const zd u0 = y[0][0] * u + y[0][1] * v, u1 = y[1][0] * u + y[1][1] * v;
       const zd r0 = (y[0][0] * a1[r] + y[0][1] * a2[r]) - th[0] * (y[0][0] * b1[r] + y[0][1] * b2[r]);
@@ -1370,7 +1847,7 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
     __syncthreads();
     {
       zd *const ys[2] = {a1, a2};
-      lu_solve_n<T, NT, 2, true>(P, A, ipiv, Lb, ys, tmp2, L.w2);
+      lu_solve_many<T, NT, 2, true>(P, A, ipiv, Lb, ys, tmp2, L.w2);
     }
     for (int r = t; r < n; r += NT) {
       x1[r] = x1[r] - a1[r] * dc[r];
@@ -1387,15 +1864,8 @@ __device__ __forceinline__ void invit2_point(const PointDev &P, int p, const cx<
     double bm = -1.0;
     int bi = 0x7fffffff;
     for (int r = t; r < n; r += NT) { const double a = abs2(x[r]); if (a > bm) { bm = a; bi = r; } }
-    s_mx[t] = bm; s_ix[t] = bi;
-    __syncthreads();
-    if (t == 0) {
-      for (int j = 1; j < NT; ++j)
-        if (s_mx[j] > bm || (s_mx[j] == bm && s_ix[j] < bi)) { bm = s_mx[j]; bi = s_ix[j]; }
-      s_ix[0] = clamp_index(bi, n);   // all-NaN vector: no entry compares greater
-    }
-    __syncthreads();
-    const zd scale = x[s_ix[0]];
+    // all-NaN vector: no entry compares greater
+    const zd scale = x[clamp_index(block_argmax<NT>(bm, bi, L.red), n)];
     __syncthreads();
     if (scale_ok(scale))
       for (int r = t; r < n; r += NT) x[r] = cdiv(x[r], scale);
@@ -1451,7 +1921,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
   extern __shared__ zd lds[];
   const int pi = order ? order[blockIdx.x] : blockIdx.x;   // largest points first
   const PointDev &P = pts[pi];
-  OpLds L(lds, P, npadmax, nymax, 1, npadmax);
+  OpLds L(lds, NT, npadmax, nymax, 1, npadmax);
   const int t = threadIdx.x, n = P.n;
   const cx<T> *A = mats + P.mat_off;
   const int *ipiv = pivs + P.piv_off;
@@ -1462,8 +1932,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
                nC = sqrt(norms[pi * 4 + 2]);
   const zd sg = P.shift;
   zd *x = L.z;
-  __shared__ double s_mx[NT];
-  __shared__ int s_ix[NT];
 
   // ---- start: x = L(sigma)^-1 L'(sigma) r
   const unsigned seed = point_seed(P);
@@ -1499,7 +1967,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     if (temporal) {
       pencil_apply<NT>(P, coef, ops, FORM_AM, sg, x, L.y, L.X1, L.X2, L.red);
       pencil_apply<NT>(P, coef, ops, FORM_BM, sg, x, L.rhs, L.X1, L.X2, L.red);
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         d3[0] = cfmac(d3[0], x[r], L.y[r]);
         d3[1] = cfmac(d3[1], x[r], L.rhs[r]);
       }
@@ -1509,7 +1977,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
       pencil_apply<NT>(P, coef, ops, FORM_C0, sg, x, L.y, L.X1, L.X2, L.red);
       pencil_apply<NT>(P, coef, ops, FORM_C1, sg, x, L.rhs, L.X1, L.X2, L.red);
       pencil_apply<NT>(P, coef, ops, FORM_C2, sg, x, L.res, L.X1, L.X2, L.red);
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         d3[0] = cfmac(d3[0], x[r], L.y[r]);
         d3[1] = cfmac(d3[1], x[r], L.rhs[r]);
         d3[2] = cfmac(d3[2], x[r], L.res[r]);
@@ -1533,14 +2001,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     // residual r = L(lambda) x into rhs
     zd part[1] = {czero<double>()};
     if (temporal) {
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         const zd v = L.y[r] - lam * L.rhs[r];
         L.rhs[r] = v;
         part[0].x += abs2(v);
       }
     } else {
       const zd l2 = lam * lam;
-      for (int r = t; r < n; r += NT) {
+      for (int r = red_first(); r < n; r += RT) {
         const zd v = L.y[r] + lam * L.rhs[r] + l2 * L.res[r];
         L.rhs[r] = v;
         part[0].x += abs2(v);
@@ -1575,15 +2043,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
   double bm = -1.0;
   int bi = 0x7fffffff;
   for (int r = t; r < n; r += NT) { const double a = abs2(x[r]); if (a > bm) { bm = a; bi = r; } }
-  s_mx[t] = bm; s_ix[t] = bi;
-  __syncthreads();
-  if (t == 0) {
-    for (int k = 1; k < NT; ++k)
-      if (s_mx[k] > bm || (s_mx[k] == bm && s_ix[k] < bi)) { bm = s_mx[k]; bi = s_ix[k]; }
-    s_ix[0] = clamp_index(bi, n);     // all-NaN vector: no entry compares greater
-  }
-  __syncthreads();
-  const zd scale = x[s_ix[0]];
+  // all-NaN vector: no entry compares greater
+  const zd scale = x[clamp_index(block_argmax<NT>(bm, bi, L.red), n)];
   __syncthreads();
   if (scale_ok(scale))
     for (int r = t; r < n; r += NT) x[r] = cdiv(x[r], scale);
@@ -1607,11 +2068,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
   // x (L.z), x2 L.res, a1 L.y, a2 L.rhs, b1 and b2 columns 2 and 3 of the
   // point's vector block, tmp2 the 2 NT entries after the operator layout.
   if (pass2 == 2 && lead2_needed(info[pi], P.itype, (rel < 1e-14) ? 0 : 2, want, P.alpha.x, lam, ff, nsolve, maxit)) {
-    zd *tmp2 = lds + op_lds_bytes(npadmax, nymax, 1, npadmax) / sizeof(zd);
+    zd *tmp2 = NT > 256 ? L.tmp : lds + op_lds_bytes(npadmax, nymax, 1, npadmax) / sizeof(zd);
     const size_t nv = P.nvec;
     invit2_point<T, NB, NT>(P, pi, mats, pivs, blks, scales, coef, ops, norms, 2 * maxit, tol, want, eval2, evec,
-                            resid2, ff2, iters, L, x, L.res, L.y, out + 2 * nv, L.rhs, out + 3 * nv, tmp2, s_mx,
-                            s_ix);
+                            resid2, ff2, iters, L, x, L.res, L.y, out + 2 * nv, L.rhs, out + 3 * nv, tmp2);
   }
 }
 
@@ -1642,17 +2102,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     if (!lead2_needed(info[p], Q.itype, flag[p], want, Q.alpha.x, eval1[p], ff1[p], iters[p], maxit1)) return;
   }
   const PointDev &P = pts[p];
-  OpLds L(lds, P, npadmax, nymax, 1, npadmax);
+  OpLds L(lds, NT, npadmax, nymax, 1, npadmax);
   zd *x1 = L.X2 + 5 * nymax;
   zd *x2 = x1 + npadmax, *a1 = x2 + npadmax, *b1 = a1 + npadmax, *a2 = b1 + npadmax, *b2 = a2 + npadmax;
   zd *tmp2 = b2 + npadmax;                     // 2 NT entries for the two-column solve
-  __shared__ double s_mx[NT];
-  __shared__ int s_ix[NT];
   zd *out = evec + P.out_off;
   for (int r = threadIdx.x; r < P.n; r += NT) x1[r] = out[r];
   __syncthreads();
   invit2_point<T, NB, NT>(P, p, mats, pivs, blks, scales, coef, ops, norms, maxit, tol, want, eval2, evec, resid2,
-                          ff2, iters, L, x1, x2, a1, b1, a2, b2, tmp2, s_mx, s_ix);
+                          ff2, iters, L, x1, x2, a1, b1, a2, b2, tmp2);
 }
 
 // Copy column sel[p] of each point's eigenvector block (P.out_off, nvec rows,

@@ -125,19 +125,50 @@ __device__ inline zd pencil_entry(const PointDev &P, const zd *__restrict__ coef
   return v;
 }
 
+// for j in [j0, n): use(j, load(j)) in ascending j, the loads of U terms issued
+// before the first is used; the rest in groups of U / 2, U / 4, ...  (In a
+// plain unrolled loop, and where a use is conditional, the compiler moves
+// each load down to its use: a memory latency per term.)
+template <int U, typename L, typename F> __device__ __forceinline__ void for_loaded(int n, L load, F use, int j0 = 0) {
+  for (; j0 + U <= n; j0 += U) {
+    decltype(load(0)) v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = load(j0 + u);
+#pragma unroll
+    for (int u = 0; u < U; ++u) use(j0 + u, v[u]);
+  }
+  if constexpr (U > 1) for_loaded<U / 2>(n, load, use, j0);
+}
+
 // ---------------------------------------------------------------------------
 // Matrix-free product y = M x for one point inside a work-group.
 // x, y: LDS vectors of P.n complex (node-major); X1, X2: LDS scratch of 5 ny.
 // All threads of the block must call it.  Padding entries are not touched.
 // ---------------------------------------------------------------------------
+// Always inlined: as a call it would give every kernel the registers and the
+// private stack of the worst case.
 template <int NT>
-__device__ void pencil_apply(const PointDev &P, const zd *__restrict__ coef, const double *__restrict__ ops, int form,
+__device__ __forceinline__ void pencil_apply(const PointDev &P, const zd *__restrict__ coef, const double *__restrict__ ops, int form,
                              zd sig, const zd *x, zd *y, zd *X1, zd *X2, zd *red) {
   const int ny = P.ny, n = P.n, t = threadIdx.x;
   const double *D1 = ops + P.op_off, *D2 = D1 + (size_t)ny * ny, *dt2w = D2 + (size_t)ny * ny;
   const bool need_d2 = (form == FORM_A0 || form == FORM_AM || form == FORM_C0 || form == FORM_SHIFTED);
   const bool need_d1 = (form != FORM_B0 && form != FORM_BM && form != FORM_C2);
-  if (need_d1 && need_d2 && 2 * ny <= NT) {
+  if constexpr (NT > 256) {
+    // a thread per (operator, variable, node), terms in the order of the
+    // branches below: 10 ny chains instead of 2 ny of five variables each (27
+    // us at ny = 96 on 256 threads, 20 here); consecutive lanes take
+    // consecutive nodes, so the operator loads coalesce and x is broadcast
+    const int nop = need_d1 ? (need_d2 ? 2 : 1) : 0;
+    for (int u = t; u < 5 * nop * ny; u += NT) {
+      const int g = u >= 5 * ny ? 1 : 0, k = (u - 5 * ny * g) / ny, i = u - 5 * ny * g - k * ny;
+      const double *D = (g ? D2 : D1) + i;
+      zd a = czero<double>();
+      for_loaded<16>(ny, [&](int j) { return D[(size_t)j * ny]; }, [&](int j, double d) { a = a + x[j * 5 + k] * d; });
+      (g ? X2 : X1)[i * 5 + k] = a;
+      if (nop == 1) X2[i * 5 + k] = czero<double>();     // read below with zero coefficients
+    }
+  } else if (need_d1 && need_d2 && 2 * ny <= NT) {
     // one half of the work-group forms X1 = D1 x, the other X2 = D2 x, one
     // node row per thread
     const int g = (t >= NT / 2) ? 1 : 0, i = t - g * (NT / 2);

@@ -71,11 +71,14 @@ __global__ void k_cheb_d2(int ny, const double *__restrict__ D1, double *__restr
   if (e >= ny * ny) return;
   const int i = e % ny, j = e / ny;
   double s = 0.0;
-  for (int k = 0; k < ny; ++k) s += D1[(size_t)k * ny + i] * D1[(size_t)j * ny + k];
+  struct D12 { double a, b; };
+  for_loaded<8>(ny, [&](int k) { return D12{D1[(size_t)k * ny + i], D1[(size_t)j * ny + k]}; },
+                [&](int, D12 d) { s += d.a * d.b; });
   D2[(size_t)j * ny + i] = s;
   if (i == ny - 1) {
     double w = 0.0;
-    for (int k = 0; k < ny - 1; ++k) w += D1[(size_t)k * ny + (ny - 1)] * D1[(size_t)j * ny + k];
+    for_loaded<8>(ny - 1, [&](int k) { return D12{D1[(size_t)k * ny + (ny - 1)], D1[(size_t)j * ny + k]}; },
+                  [&](int, D12 d) { w += d.a * d.b; });
     dt2w[j] = w;
   }
 }
@@ -88,15 +91,14 @@ __global__ void k_cheb_sums(int ny, const double *__restrict__ D1, const double 
   double *sums = dt2w + ny;
   for (int i = threadIdx.x; i < ny; i += blockDim.x) {
     double a = 0.0, b = 0.0, c = 0.0;
-    for (int j = 0; j < ny; ++j) {
-      const double d1 = D1[(size_t)j * ny + i], d2 = D2[(size_t)j * ny + i];
-      a += d1 * d1; b += d2 * d2; c += d1 * d2;
-    }
+    struct D12 { double a, b; };
+    for_loaded<8>(ny, [&](int j) { return D12{D1[(size_t)j * ny + i], D2[(size_t)j * ny + i]}; },
+                  [&](int, D12 d) { a += d.a * d.a; b += d.b * d.b; c += d.a * d.b; });
     sums[i] = a; sums[ny + i] = b; sums[2 * ny + i] = c;
   }
   if (threadIdx.x == 0) {
     double s = 0.0;
-    for (int j = 0; j < ny; ++j) s += dt2w[j] * dt2w[j];
+    for_loaded<16>(ny, [&](int j) { return dt2w[j]; }, [&](int, double d) { s += d * d; });
     sums[3 * ny] = s;
   }
 }
