@@ -487,9 +487,9 @@ int launch_lu_step(stab_ctx *c, hipStream_t s, int R, const LuStep &st, const in
   cx<T> *mats = (cx<T> *)B.mats, *blks = (cx<T> *)B.blks;
   if (st.npanel > 0) {
     switch (R) {
-      case 1: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 1, 16>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
-      case 2: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 2, 16>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
-      case 3: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 3, 16>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
+      case 1: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 1>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
+      case 2: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 2>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
+      case 3: hipLaunchKernelGGL((k_lu_panel<T, NB, NT, 3>), dim3(st.npanel), dim3(NT), 0, s, B.pts, mats, B.pivs, blks, B.info, order, left, st.K0); break;
       default: return fail(c, STAB_E_ARG, "matrix order too large for the LU kernel (%d panel rows)", R);
     }
     HIPCHECK(c, hipGetLastError());

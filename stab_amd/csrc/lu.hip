@@ -4,10 +4,12 @@
 // Columns are taken in blocks of KB = 64 (the last may be 32 wide).  Inside a
 // block, panels of NB columns (16 in FP32, 8 in FP64) are factored with their rows in registers
 // of the threads that own them (row r belongs to thread r % NT), so the pivot
-// search, the row interchanges inside the panel and the rank-1 updates never
-// touch memory; each panel then updates the rest of its block column (all
-// rows) in strips of SW columns, applying its interchanges through LDS and
-// forming its rows of U as inv(L11) * A12.  When the block column is done:
+// search and the rank-1 updates never touch memory.  Rows do not move while a
+// block is factored: each thread tracks the position its rows would have
+// after the interchanges so far (the pivot search compares positions, so the
+// choice is the one of moved rows).  Each panel updates the rest of its block
+// column in place, its rows of U being inv(L11) * A12.  When the block column
+// is done its rows are put in their final order in one pass, and:
 //   * its net row permutation is applied once to the trailing columns and,
 //     for the LAPACK form only (left = 1), to the columns left of it;
 //     otherwise it is stored as the block's interchange record for the solves,
@@ -27,6 +29,8 @@
 // row order and perm (ipiv + n, P as a row list) is stored too; with left = 0
 // the columns left of each block keep their rows (mode 1).
 #include "common.h"
+#include <type_traits>
+#include <utility>
 
 // 16 x 16 x 4 MFMA: D[m][n] += sum_k A[m][k] B[k][n]; lane l supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16].  Accumulator register i of lane l
@@ -58,23 +62,58 @@ __host__ __device__ inline long long blk_elems(int npad, int bs) {
   return 2LL * nblk * bs * bs;
 }
 
-// Net permutation of the interchanges ipiv[k0 .. k0+w) (absolute rows, each
-// >= its step): touched rows srow[e] receive the input row sorig[e];
-// returns the number of touched rows (<= 2 w).  One thread; slot[] (one
-// entry per row, -1 when the row is not in the list) finds a row's entry in
-// O(1) and is -1 again on return.
-__device__ inline int net_perm(const int *ipiv, int k0, int w, int *srow, int *sorig, int *slot) {
-  int ns = 0;
-  for (int c = 0; c < w; ++c) {
-    const int a = k0 + c, b = ipiv[c];
-    if (a == b) continue;
-    int ia = slot[a], ib = slot[b];
-    if (ia < 0) { ia = ns; srow[ns] = a; sorig[ns] = a; slot[a] = ns; ++ns; }
-    if (ib < 0) { ib = ns; srow[ns] = b; sorig[ns] = b; slot[b] = ns; ++ns; }
-    const int tmp = sorig[ia]; sorig[ia] = sorig[ib]; sorig[ib] = tmp;
+// f(0), ..., f(N - 1) with the index a compile-time constant in each
+template <int... I, typename F> __device__ __forceinline__ void static_for_(std::integer_sequence<int, I...>, const F &f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F> __device__ __forceinline__ void static_for(const F &f) {
+  static_for_(std::make_integer_sequence<int, N>{}, f);
+}
+
+// Order the LDS accesses of one wave's lanes.
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The wave's arg-max of (v, i): larger v, the lower i among equal v; v is a
+// magnitude or -1 (no candidate).  The index comes back for the whole wave.
+// Floats of these values order as their bits do, so the maximum is six integer
+// DPP maxima of the (high) words; only where more than one lane holds it are
+// the low words, then the indexes, compared.
+__device__ inline int wave_max(int x) {
+  constexpr int LOW = (int)0x80000000;
+#define STAB_MAX_STEP(CTRL, RM) x = max(__builtin_amdgcn_update_dpp(LOW, x, CTRL, RM, 0xF, false), x);
+  STAB_MAX_STEP(0x111, 0xF) STAB_MAX_STEP(0x112, 0xF) STAB_MAX_STEP(0x114, 0xF) STAB_MAX_STEP(0x118, 0xF)
+  STAB_MAX_STEP(0x142, 0xA) STAB_MAX_STEP(0x143, 0xC)
+#undef STAB_MAX_STEP
+  return lane63(x);
+}
+__device__ inline int wave_best(int hi, unsigned lo, int i) {
+  unsigned long long at = __ballot(hi == wave_max(hi));
+  if (__builtin_expect((at & (at - 1)) != 0, 0)) {
+    const int key = ((at >> (threadIdx.x & 63)) & 1ull) ? (int)(lo ^ 0x80000000u) : (int)0x80000000;
+    at &= __ballot(key == wave_max(key));
+    const int mi = ((at >> (threadIdx.x & 63)) & 1ull) ? ~i : (int)0x80000000;
+    return ~wave_max(mi);
   }
-  for (int e = 0; e < ns; ++e) slot[srow[e]] = -1;
-  return ns;
+  return __builtin_amdgcn_readlane(i, __builtin_ctzll(at));
+}
+__device__ inline int wave_best(float v, int i) { return wave_best(__float_as_int(v), 0u, i); }
+__device__ inline int wave_best(double v, int i) {
+  const long long b = __double_as_longlong(v);
+  return wave_best((int)(b >> 32), (unsigned)b, i);
+}
+
+// 1 / b as cdiv(1, b) rounds it (zeros keep the signs that gives them), on one
+// path: the larger component divides.
+template <typename T> __device__ inline cx<T> crecip(cx<T> b) {
+  const bool ge = fabs(b.x) >= fabs(b.y);
+  const T big = ge ? b.x : b.y, sm = ge ? b.y : b.x;
+  const T r = sm / big, d = fma(sm, r, big);
+  const T nr = sizeof(T) == 4 ? -r : (T)0 - r;
+  return mk<T>((ge ? (T)1 : r + (T)0) / d, (ge ? nr : (T)-1) / d);
 }
 
 // The batched LU in two launches per 64-column block (K0 = 0, 64, ...) over
@@ -91,7 +130,14 @@ __device__ inline int net_perm(const int *ipiv, int k0, int w, int *srow, int *s
 // Split this way, the strips of one matrix run on several CUs at once and the
 // latency-bound panel steps of some matrices overlap the matrix-core updates
 // of others; the arithmetic is that of one work-group doing both in turn.
-template <typename T, int NB, int NT, int R, int SW>
+// A lone panel is bound by latency and by what one wave per SIMD issues: 64
+// columns, each an arg-max, a publication through LDS, one barrier and a
+// rank-1 update.  With rows that moved at every pivot, serial net permutations
+// and strips of 16 columns loaded, updated and stored in turn, the panels of
+// one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.91
+// and 1.37 (256 such matrices: 1.88 and 2.92 ms, now 1.12 and 1.90); 0.38 and
+// 0.41 ms of that are the columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.
+template <typename T, int NB, int NT, int R>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 && NT == 256 ? 3 : 2))) void k_lu_panel(const PointDev *__restrict__ pts, cx<T> *__restrict__ mats,
                                                  int *__restrict__ pivs, cx<T> *__restrict__ blks,
                                                  int *__restrict__ info, const int *__restrict__ order, int left,
@@ -105,418 +151,425 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 && NT
   if (K0 >= n) return;
   C *A = mats + P.mat_off;
   int *ipiv = pivs + P.piv_off;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   constexpr int NW = NT / 64;
-  constexpr int KB = 64, SU = 2 * KB * 16;
+  constexpr int KB = 64, SU = 2 * KB * 16, WS = KB - NB;    // WS: widest rest of the block column
+  constexpr int NONE = 0x7fffffff;
   static_assert(KB % NB == 0, "panel width must divide the block width");
   static_assert(LU_PREC == 1 + 4 * KB, "interchange record: count, 2 KB rows, 2 KB sources");
   static_assert(LU_TREC == 1 + 3 * KB, "trailing record: count, KB top sources, KB out rows, KB out sources");
 
   // double-buffered by column parity: a column's slots are rewritten two
   // columns later, after a barrier every wave passes only once it has read
-  // them.  s_cand2: each wave's best candidate row, s_crow2: the row of the
-  // diagonal; both are published before the column's one barrier.
-  __shared__ C s_cand2[2][NW][NB], s_crow2[2][NB];
-  __shared__ T s_rv2[2][NW];
-  __shared__ int s_ri2[2][NW];
+  // them.  Each wave publishes its best candidate and that row before the
+  // column's one barrier.
+  struct __attribute__((aligned(16))) Best { C inv; T v; int i; };   // a candidate: reciprocal, magnitude, position
+  __shared__ C s_cand2[2][NW][NB];
+  __shared__ Best s_best2[2][NW];
   __shared__ C s_blk[NB * NB];
   __shared__ C s_linv[NB * NB];           // inv(L11) of the current panel
-  __shared__ int s_piv[KB];
+  __shared__ int s_top[NB];               // rows (slots) of the panel's pivots
   __shared__ int s_srow[2 * KB], s_sorig[2 * KB];
-  __shared__ int s_slot[1280];            // net_perm's row map (npad <= 1280)
-  __shared__ int s_topsrc[KB], s_outrow[KB], s_outsrc[KB];
-  __shared__ int s_nout, s_ns;
-  __shared__ C s_stage[2 * NB * SW];
-  __shared__ C s_u12[NB * SW];
-  // packed strictly lower L11 for X (KB (KB - 1) / 2 entries), staging of the
-  // left-column interchanges (at most 2 KB rows x 16 columns), the final row list
+  __shared__ int s_cnt[2][NW * R];
+  __shared__ C s_u12[NB * WS];
+  // staged A12 of the panel's pivot rows, then L21 in operand order (FP32);
+  // packed strictly lower L11 for X (KB (KB - 1) / 2 entries); the left-column
+  // interchanges (at most 2 KB rows x 16 columns); the final row list
   __shared__ C s_u[SU];
+  static_assert(NB * WS <= SU, "A12 fits in s_u");
 
   C Pn[R][NB];
+  int pos[R];                              // position of row K0 + t + j NT; NONE past the matrix
+#pragma unroll
+  for (int j = 0; j < R; ++j) pos[j] = (K0 + t + j * NT < n) ? K0 + t + j * NT : NONE;
+  int mypiv = 0;                           // the pivot of column K0 + t
   int myinfo = (K0 == 0) ? 0 : info[pi];   // the first zero pivot of the earlier blocks
-  for (int r = t; r < 1280; r += NT) s_slot[r] = -1;
-  __syncthreads();
 
-  {
-    const int kb = min(KB, n - K0);       // 64, or 32 for the last block (n is a multiple of 32)
-    const int kend = K0 + kb;
-    for (int k0 = K0; k0 < kend; k0 += NB) {
-      // ---- load the panel rows owned by this thread
+  const int kb = min(KB, n - K0);       // 64, or 32 for the last block (n is a multiple of 32)
+  const int kend = K0 + kb;
+  // row j of this thread (rows past the matrix: row K0), and its entry in a
+  // column.  The column's address is uniform and passes through the asm so that
+  // it stays a scalar of its own: 2 R NB whole addresses per lane, kept from the
+  // loads to the stores, would spill.
+  auto slot = [&](int j) { return K0 + t + j * NT < n ? K0 + t + j * NT : K0; };
+  auto at = [&](int col, unsigned row) -> C & {
+    char *cp = reinterpret_cast<char *>(A + (size_t)col * lda);
+    asm volatile("" : "+s"(cp));
+    return *reinterpret_cast<C *>(cp + row * (unsigned)sizeof(C));
+  };
+  for (int k0 = K0; k0 < kend; k0 += NB) {
+    // ---- load the panel (rows that were pivots earlier carry values that are
+    // not used)
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int c = 0; c < NB; ++c) Pn[j][c] = at(k0 + c, slot(j));
+    // ---- factor the panel; every register index is static, so the rank-1
+    // updates touch only the columns right of the pivot
+    static_for<NB>([&](auto cs) {
+      constexpr int c = cs;
+      const int col = k0 + c;
+      T lv = (T)-1;
+      int li = NONE;
+      C lc = czero<T>();
 #pragma unroll
       for (int j = 0; j < R; ++j) {
-        const int r = K0 + t + j * NT;
-#pragma unroll
-        for (int c = 0; c < NB; ++c)
-        {
-          // unconditional load from a row in range, then select: a load under
-          // a divergent branch waits for its data before the branch joins
-          const bool ok = r >= k0 && r < n;
-          const C v = A[(size_t)(k0 + c) * lda + (ok ? r : k0)];
-          Pn[j][c] = ok ? v : czero<T>();
-        }
+        const T v = cabs1(Pn[j][c]);
+        // a NaN never becomes a candidate; among equal magnitudes the lower position
+        const bool up = (pos[j] >= col) & (pos[j] < NONE) & ((v > lv) | ((v == lv) & (pos[j] < li)));
+        lv = up ? v : lv;
+        li = up ? pos[j] : li;
+        lc = mk<T>(up ? Pn[j][c].x : lc.x, up ? Pn[j][c].y : lc.y);
       }
-      // ---- factor the panel.  Every register access below has compile-time
-      // column indices (with predicates when the loop is not unrolled), so Pn
-      // stays in VGPRs.  FP32 unrolls the column loop, so the rank-1 updates
-      // touch only the columns right of the pivot; FP64 (more registers per
-      // entry) keeps it rolled.
-      constexpr int PANEL_UNROLL = sizeof(T) == 4 ? NB : 1;
-#pragma unroll PANEL_UNROLL
-      for (int c = 0; c < NB; ++c) {
-        const int col = k0 + c;
-        C *s_crow = s_crow2[c & 1];
-        T *s_rv = s_rv2[c & 1];
-        int *s_ri = s_ri2[c & 1];
-        T best = (T)-1;
-        int bi = 0x7fffffff;
+      // every lane takes the reciprocal of its own candidate: a division is a
+      // chain of dependent steps as the wave's arg-max is, and the two run
+      // interleaved instead of one after the other
+      const C rc = crecip(lc);
+      const int bi = wave_best(lv, li);
+      if (li == bi) {                       // the lane that holds the row at position bi (all, where none does)
+        s_best2[c & 1][wv] = Best{rc, lv, li};
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-          const int r = K0 + t + j * NT;
-          C pc = czero<T>();
+          if (pos[j] == bi) {
 #pragma unroll
-          for (int cc = 0; cc < NB; ++cc) if (cc == c) pc = Pn[j][cc];
-          if (r >= col && r < n) {
-            const T v = cabs1(pc);
-            if (v > best) { best = v; bi = r; }
-          }
-        }
-        // best is -1 or a magnitude (a NaN one never replaces it), so the
-        // wave's arg-max is well defined
-        wave_argmax(best, bi);
-        // publish the wave's candidate (value, row index, the row itself) and
-        // the diagonal row; one barrier then serves the pivot choice and the
-        // interchange.  The wave's candidate rows are its own rows, so the
-        // owner of row bi is a lane of this wave.
-        if (lane == 0) { s_rv[wv] = best; s_ri[wv] = bi; }
-        const int cj = (col - K0) / NT, bj = (bi < n) ? (bi - K0) / NT : -1;
-#pragma unroll
-        for (int j = 0; j < R; ++j) {
-          if (j == bj && ((bi - K0) % NT) == t) {
-#pragma unroll
-            for (int cc = 0; cc < NB; ++cc) s_cand2[c & 1][wv][cc] = Pn[j][cc];
-          }
-          if (j == cj && ((col - K0) % NT) == t) {
-#pragma unroll
-            for (int cc = 0; cc < NB; ++cc) s_crow[cc] = Pn[j][cc];
-          }
-        }
-        __syncthreads();
-        best = s_rv[0]; bi = s_ri[0];
-        int wb = 0;
-#pragma unroll
-        for (int w = 1; w < NW; ++w) {
-          if (s_rv[w] > best || (s_rv[w] == best && s_ri[w] < bi)) { best = s_rv[w]; bi = s_ri[w]; wb = w; }
-        }
-        // no finite candidate (NaN column): keep the diagonal so every index stays in range
-        const bool found = (bi >= col && bi < n);
-        const int p = found ? bi : col;
-        const C *s_prow = found ? s_cand2[c & 1][wb] : s_crow;
-        const int pj = (p - K0) / NT;
-        if (p != col) {
-#pragma unroll
-          for (int j = 0; j < R; ++j) {
-            if (j == pj && ((p - K0) % NT) == t) {
-#pragma unroll
-              for (int cc = 0; cc < NB; ++cc) Pn[j][cc] = s_crow[cc];
-            }
-            if (j == cj && ((col - K0) % NT) == t) {
-#pragma unroll
-              for (int cc = 0; cc < NB; ++cc) Pn[j][cc] = s_prow[cc];
-            }
-          }
-        }
-        const C piv = s_prow[c];
-        if (t == 0) s_piv[col - K0] = p;
-        if (piv.x == (T)0 && piv.y == (T)0) {
-          if (myinfo == 0) myinfo = col + 1;
-        } else {
-          const C inv = cdiv(mk<T>(1, 0), piv);
-#pragma unroll
-          for (int j = 0; j < R; ++j) {
-            const int r = K0 + t + j * NT;
-            if (r > col && r < n) {
-              C l = czero<T>();
-#pragma unroll
-              for (int cc = 0; cc < NB; ++cc) if (cc == c) l = Pn[j][cc];
-              l = l * inv;
-#pragma unroll
-              for (int cc = 0; cc < NB; ++cc) {
-                if (cc == c) Pn[j][cc] = l;
-                else if (cc > c) Pn[j][cc] = cfms(Pn[j][cc], l, s_prow[cc]);
-              }
-            }
-          }
-        }
-      }
-      // ---- write the factored panel back; stage the diagonal block
-#pragma unroll
-      for (int j = 0; j < R; ++j) {
-        const int r = K0 + t + j * NT;
-        if (r >= k0 && r < n) {
-#pragma unroll
-          for (int c = 0; c < NB; ++c) A[(size_t)(k0 + c) * lda + r] = Pn[j][c];
-          if (r < k0 + NB) {
-#pragma unroll
-            for (int c = 0; c < NB; ++c) s_blk[(r - k0) * NB + c] = Pn[j][c];
+            for (int cc = c + 1; cc < NB; ++cc) s_cand2[c & 1][wv][cc] = Pn[j][cc];
           }
         }
       }
       __syncthreads();
-      // ---- inv(L11) (unit lower), one column per thread, the column in
-      // registers (the terms k < c vanish: x[k] = 0 there)
-      if (t < NB) {
-        const int c = t;
+      Best b = s_best2[c & 1][0];
+      int wb = 0;
+#pragma unroll
+      for (int w = 1; w < NW; ++w) {
+        const Best o = s_best2[c & 1][w];
+        const bool up = (o.v > b.v) | ((o.v == b.v) & (o.i < b.i));
+        b.inv = mk<T>(up ? o.inv.x : b.inv.x, up ? o.inv.y : b.inv.y);
+        b.v = up ? o.v : b.v;
+        b.i = up ? o.i : b.i;
+        wb = up ? w : wb;
+      }
+      if (__builtin_expect(__builtin_amdgcn_readfirstlane(b.i) == NONE, 0)) {
+        // no candidate but NaN: keep the diagonal, whose reciprocal is NaN
+        b.i = col;
+        wb = 0;
+        b.inv = mk<T>((T)__builtin_nan(""), (T)__builtin_nan(""));
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          if (pos[j] == col) {
+#pragma unroll
+            for (int cc = c + 1; cc < NB; ++cc) s_cand2[c & 1][0][cc] = Pn[j][cc];
+          }
+        }
+        __syncthreads();
+      }
+      const int p = b.i;
+      mypiv = (t == col - K0) ? p : mypiv;
+      const bool zero = b.v == (T)0;
+      myinfo = (zero & (myinfo == 0)) ? col + 1 : myinfo;
+      C u[NB];
+#pragma unroll
+      for (int cc = c + 1; cc < NB; ++cc) u[cc] = s_cand2[c & 1][wb][cc];
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        pos[j] = (pos[j] == p) ? col : (pos[j] == col ? p : pos[j]);
+        if ((pos[j] > col) & (pos[j] < NONE) & !zero) {
+          const C l = Pn[j][c] * b.inv;
+          Pn[j][c] = l;
+#pragma unroll
+          for (int cc = c + 1; cc < NB; ++cc) Pn[j][cc] = cfms(Pn[j][cc], l, u[cc]);
+        }
+      }
+    });
+    // ---- write the factored panel back (rows still in place); stage the
+    // diagonal block
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      if (pos[j] >= k0 && pos[j] < NONE) {
+#pragma unroll
+        for (int c = 0; c < NB; ++c) at(k0 + c, slot(j)) = Pn[j][c];
+        if (pos[j] < k0 + NB) {
+          s_top[pos[j] - k0] = slot(j);
+#pragma unroll
+          for (int c = 0; c < NB; ++c) s_blk[(pos[j] - k0) * NB + c] = Pn[j][c];
+        }
+      }
+    }
+    __syncthreads();
+    const int c0 = k0 + NB, w = kend - c0;      // the rest of the block column
+    if (w <= 0) break;
+    // ---- A12: the pivot rows of the rest, staged by the waves after the
+    // first, while 16 (8) lanes of the first form inv(L11) (unit lower), one
+    // column per lane in registers, term k of every row as soon as x[k] is known
+    // (the terms k < c vanish: x[k] = 0 there)
+    if (wv == 0) {
+      if (lane < NB) {
+        const int c = lane;
         C x[NB];
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          C s = (i == c) ? mk<T>(1, 0) : czero<T>();
+        for (int i = 0; i < NB; ++i) x[i] = mk<T>((T)(i == c), 0);
+        static_for<NB - 1>([&](auto ks) {
+          constexpr int k = ks;
+          x[k] = mk<T>(k < c ? (T)0 : x[k].x, k < c ? (T)0 : x[k].y);
 #pragma unroll
-          for (int k = 0; k < i; ++k) s = cfms(s, (k >= c) ? s_blk[i * NB + k] : czero<T>(), x[k]);
-          x[i] = (i < c) ? czero<T>() : s;
-        }
+          for (int i = k + 1; i < NB; ++i) {
+            const C l = s_blk[i * NB + k];
+            x[i] = cfms(x[i], mk<T>(k < c ? (T)0 : l.x, k < c ? (T)0 : l.y), x[k]);
+          }
+        });
 #pragma unroll
         for (int i = 0; i < NB; ++i) s_linv[i * NB + c] = x[i];
       }
-      __syncthreads();
-      if (t < NB) ipiv[k0 + t] = s_piv[k0 - K0 + t];
-      // ---- net permutation of the panel's interchanges: rows of the panel
-      // top and the rows below it that change
-      if (t == 0) {
-        const int ns = net_perm(s_piv + (k0 - K0), k0, NB, s_srow, s_sorig, s_slot);
-        for (int c = 0; c < NB; ++c) s_topsrc[c] = k0 + c;
-        int no = 0;
-        for (int e = 0; e < ns; ++e) {
-          const int row = s_srow[e];
-          if (row < k0 + NB) s_topsrc[row - k0] = s_sorig[e];
-          else if (s_sorig[e] != row) { s_outrow[no] = row; s_outsrc[no] = s_sorig[e]; ++no; }
-        }
-        s_nout = no;
-        s_ns = ns;
+    } else {
+      for (int e = t - 64; e < NB * w; e += NT - 64) {
+        const int i = e % NB, cc = e / NB;
+        s_u[i * WS + cc] = A[(size_t)(c0 + cc) * lda + s_top[i]];
       }
-      __syncthreads();
-      // ---- the rest of the block column, in strips of SW columns
-      const int nout = s_nout, nslot = NB + nout;
-      const C *Li = s_linv;
-      for (int c0 = k0 + NB; c0 < kend; c0 += SW) {
-        const int sw = min(SW, kend - c0);      // strips never cross the block end
-        for (int e = t; e < nslot * sw; e += NT) {
-          const int slot = e % nslot, cc = e / nslot;
-          const int src = (slot < NB) ? s_topsrc[slot] : s_outsrc[slot - NB];
-          s_stage[slot * SW + cc] = A[(size_t)(c0 + cc) * lda + src];
-        }
-        __syncthreads();
-        for (int e = t; e < nout * sw; e += NT) {
-          const int o = e % nout, cc = e / nout;
-          A[(size_t)(c0 + cc) * lda + s_outrow[o]] = s_stage[(NB + o) * SW + cc];
-        }
-        for (int e = t; e < NB * sw; e += NT) {
-          const int i = e / sw, cc = e - i * sw;
-          C u = czero<T>();
-          for (int k = 0; k <= i; ++k) u = cfma(u, Li[i * NB + k], s_stage[k * SW + cc]);
-          s_u12[i * SW + cc] = u;
-          A[(size_t)(c0 + cc) * lda + k0 + i] = u;
-        }
-        __syncthreads();
-        // A22 strip -= L21 U12.  FP32: on the matrix cores, as the trailing
-        // kernel does it (C tile = the update transposed: lane l holds strip
-        // columns 4 (l / 16) + i of row r0 + l % 16), one 16-row tile at a
-        // time; the B operand L21(r0 + l % 16, 4 s + l / 16) belongs to
-        // another lane of the same wave, so each wave stages the L21 rows of
-        // two of its tiles (32 rows x NB) in its quarter of s_u, which the
-        // strips do not otherwise use, and reads them back in operand
-        // order.  Tiles are whole: rows below the panel start at k0 + NB, a
-        // multiple of 16, and n is a multiple of 32.
-        const int wrow = t - lane;
-        if constexpr (sizeof(T) == 4 && SW == 16 && NB == 16 && NT == 64 * NW && 32 * NB * NW <= SU) {
-          typedef typename Mfma<T>::v4 v4;
-          C *lst = s_u + (size_t)wv * 32 * NB;
+    }
+    __syncthreads();
+    for (int e = t; e < NB * w; e += NT) {
+      const int cc = e / NB, i = e - cc * NB;     // consecutive lanes: rows of one column
+      C u = czero<T>();
 #pragma unroll
-          for (int j = 0; j < R; ++j) {
-            const int w0 = K0 + wrow + j * NT;
-            if (w0 >= n || w0 + 63 < k0 + NB) continue;           // wave-uniform
+      for (int k = 0; k < NB; ++k) {
+        const C v = s_u[k * WS + cc];
+        if (k <= i) u = cfma(u, s_linv[i * NB + k], v);
+      }
+      s_u12[i * WS + cc] = u;
+      A[(size_t)(c0 + cc) * lda + s_top[i]] = u;
+    }
+    __syncthreads();
+    // ---- A22 -= L21 U12 on the rows below the panel, wherever they are.
+    if constexpr (sizeof(T) == 4 && NB == 16 && 32 * NB * NW <= SU) {
+      // FP32, on the matrix cores, as the trailing kernel does it (C tile = the
+      // update transposed: lane l holds columns 4 (l / 16) + i of row r0 + l % 16).
+      // The B operand L21(r0 + l % 16, 4 s + l / 16) belongs to another lane of
+      // the wave, so each wave stages the L21 rows of two tiles (32 rows x NB)
+      // in its part of s_u and reads them back in operand order; the column
+      // tiles of a row tile are loaded together.  Rows at or above the panel
+      // are computed with the others and not stored.
+      typedef typename Mfma<T>::v4 v4;
+      C *lst = s_u + (size_t)wv * 32 * NB;
+      const int nct = w / 16;
+      static_for<R>([&](auto js) {
+        constexpr int j = js;
+        const int w0 = K0 + 64 * wv + j * NT;
+        const unsigned long long live = __ballot(pos[j] >= c0 && pos[j] < NONE);
 #pragma unroll 1
-            for (int half = 0; half < 2; ++half) {
-              const int rb = w0 + 32 * half;                       // first row of the tile pair
-              if (rb >= n || rb + 31 < k0 + NB) continue;          // wave-uniform
-              if ((lane >> 5) == half) {
+        for (int half = 0; half < 2; ++half) {
+          const unsigned lm = (unsigned)(live >> (32 * half));
+          if (lm == 0) continue;                                   // wave-uniform
+          wave_lds_order();
+          if ((lane >> 5) == half) {
 #pragma unroll
-                for (int k = 0; k < NB; ++k) lst[(lane & 31) * NB + k] = Pn[j][k];
+            for (int k = 0; k < NB; ++k) lst[(lane & 31) * NB + k] = Pn[j][k];
+          }
+          wave_lds_order();
+#pragma unroll 1
+          for (int a = 0; a < 2; ++a) {
+            const unsigned am = (lm >> (16 * a)) & 0xffffu;
+            if (am == 0) continue;                                 // wave-uniform
+            const bool st_ok = (am >> (lane & 15)) & 1u;
+            const int r0 = w0 + 32 * half + 16 * a;
+            C *Ab = A + (size_t)(c0 + 4 * (lane >> 4)) * lda + r0 + (lane & 15);
+            v4 dr[WS / 16], di[WS / 16];
+#pragma unroll
+            for (int ct = 0; ct < WS / 16; ++ct)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const C x = Ab[(size_t)(min(ct, nct - 1) * 16 + i) * lda];
+                dr[ct][i] = x.x;
+                di[ct][i] = x.y;
               }
-              __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-              __builtin_amdgcn_wave_barrier();
-              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll 1
-              for (int a = 0; a < 2; ++a) {
-                const int r0 = rb + 16 * a;
-                if (r0 >= n || r0 < k0 + NB) continue;               // wave-uniform
-                C *Ab = A + (size_t)(c0 + 4 * (lane >> 4)) * lda + r0 + (lane & 15);
-                v4 dr, di;
+            C l[NB / 4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                  const C x = Ab[(size_t)i * lda];
-                  dr[i] = x.x;
-                  di[i] = x.y;
-                }
+            for (int st = 0; st < NB / 4; ++st) l[st] = lst[(16 * a + (lane & 15)) * NB + 4 * st + (lane >> 4)];
 #pragma unroll
-                for (int st = 0; st < NB / 4; ++st) {
-                  const C l = lst[(16 * a + (lane & 15)) * NB + 4 * st + (lane >> 4)];
-                  const C u = s_u12[(4 * st + (lane >> 4)) * SW + (lane & 15)];
-                  const T nur = -u.x, ui = u.y, nui = -u.y;
-                  dr = Mfma<T>::mac(nur, l.x, dr);
-                  dr = Mfma<T>::mac(ui, l.y, dr);
-                  di = Mfma<T>::mac(nui, l.x, di);
-                  di = Mfma<T>::mac(nur, l.y, di);
-                }
+            for (int ct = 0; ct < WS / 16; ++ct) {
+              if (ct >= nct) break;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) Ab[(size_t)i * lda] = mk<T>(dr[i], di[i]);
+              for (int st = 0; st < NB / 4; ++st) {
+                const C u = s_u12[(4 * st + (lane >> 4)) * WS + ct * 16 + (lane & 15)];
+                const T nur = -u.x, ui = u.y, nui = -u.y;
+                dr[ct] = Mfma<T>::mac(nur, l[st].x, dr[ct]);
+                dr[ct] = Mfma<T>::mac(ui, l[st].y, dr[ct]);
+                di[ct] = Mfma<T>::mac(nui, l[st].x, di[ct]);
+                di[ct] = Mfma<T>::mac(nur, l[st].y, di[ct]);
               }
-              __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-              __builtin_amdgcn_wave_barrier();
-              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+              if (st_ok) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) Ab[(size_t)(ct * 16 + i) * lda] = mk<T>(dr[ct][i], di[ct][i]);
+              }
             }
           }
-          __syncthreads();
-          continue;
         }
-        // VALU (FP64): one row slot at a time with G columns of independent
-        // accumulators; a wave skips the slots in which none of its 64 rows
-        // is below the panel and inside the matrix (the third slot of
-        // matrices of order <= 2 NT, for instance)
-        constexpr int G = (R >= 2) ? 2 : 4;
+      });
+    } else {
+      // FP64 (and 512 threads, whose staging would not fit in s_u), on the VALU
+      // (the FP64 matrix cores give the same sums in 1.42 ms against 1.37):
+      // G columns of a row at a time, the next group's entries loaded while one
+      // is computed
+      constexpr int G = 4;
+      static_for<R>([&](auto js) {
+        constexpr int j = js;
+        if (__ballot(pos[j] >= c0 && pos[j] < NONE) == 0) return;
+        const bool live = pos[j] >= c0 && pos[j] < NONE;
+        C nx[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) nx[q] = at(c0 + q, slot(j));
 #pragma unroll 1
-        for (int cg = 0; cg < sw; cg += G) {
+        for (int cg = 0; cg < w; cg += G) {
+          C acc[G];
 #pragma unroll
-          for (int j = 0; j < R; ++j) {
-            const int w0 = K0 + wrow + j * NT;
-            if (w0 >= n || w0 + 63 < k0 + NB) continue;
-            const int r = K0 + t + j * NT;
-            const bool live = (r >= k0 + NB && r < n);
-            C acc[G];
+          for (int q = 0; q < G; ++q) acc[q] = nx[q];
 #pragma unroll
-            for (int q = 0; q < G; ++q) {
-              const C v = A[(size_t)(c0 + cg + q) * lda + (live ? r : k0)];
-              acc[q] = live ? v : czero<T>();
-            }
+          for (int q = 0; q < G; ++q) nx[q] = at(c0 + min(cg + G, w - G) + q, slot(j));
 #pragma unroll
-            for (int k = 0; k < NB; ++k) {
+          for (int k = 0; k < NB; ++k)
 #pragma unroll
-              for (int q = 0; q < G; ++q) acc[q] = cfms(acc[q], Pn[j][k], s_u12[k * SW + cg + q]);
-            }
-            if (live) {
+            for (int q = 0; q < G; ++q) acc[q] = cfms(acc[q], Pn[j][k], s_u12[k * WS + cg + q]);
+          if (live) {
 #pragma unroll
-              for (int q = 0; q < G; ++q) A[(size_t)(c0 + cg + q) * lda + r] = acc[q];
-            }
+            for (int q = 0; q < G; ++q) at(c0 + cg + q, slot(j)) = acc[q];
           }
         }
-        __syncthreads();
-      }
-      // ---- the panel's interchanges on the block's columns left of it, so the
-      // block's L is in one row order when the block is done
-      const int ns = s_ns;
-      if (ns > 0 && k0 > K0) {
-        for (int c0 = K0; c0 < k0; c0 += SW) {
-          const int w = min(SW, k0 - c0);
-          for (int e = t; e < ns * w; e += NT) {
-            const int slot = e % ns, cc = e / ns;
-            s_stage[slot * SW + cc] = A[(size_t)(c0 + cc) * lda + s_sorig[slot]];
-          }
-          __syncthreads();
-          for (int e = t; e < ns * w; e += NT) {
-            const int slot = e % ns, cc = e / ns;
-            A[(size_t)(c0 + cc) * lda + s_srow[slot]] = s_stage[slot * SW + cc];
-          }
-          __syncthreads();
-        }
-      }
-    }  // panels of the block
+      });
+    }
+    __syncthreads();
+  }  // panels of the block
 
-    // ---- net permutation of the whole block: top rows K0 .. kend take the
-    // input rows s_topsrc[], rows below take s_outsrc[] (always input rows of
-    // the block top); s_srow/s_sorig list every touched row
-    if (t == 0) {
-      const int ns = net_perm(s_piv, K0, kb, s_srow, s_sorig, s_slot);
-      for (int c = 0; c < kb; ++c) s_topsrc[c] = K0 + c;
-      int no = 0;
-      for (int e = 0; e < ns; ++e) {
-        const int row = s_srow[e];
-        if (row < kend) s_topsrc[row - K0] = s_sorig[e];
-        else if (s_sorig[e] != row) { s_outrow[no] = row; s_outsrc[no] = s_sorig[e]; ++no; }
+  // ---- the interchanges: ipiv, and the block's net permutation (position
+  // pos[j] receives row slot(j)) as the record of the forward solves (every row
+  // that moves; read in pivot mode 1) and the trailing record of the update
+  // kernel (the input row of each block-top row, the rows below that change).
+  // List places in row order: counts per (j, wave), then ballot ranks.
+  if (t < kb) ipiv[K0 + t] = mypiv;
+  unsigned long long mm[R], mo[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const bool moved = pos[j] < NONE && pos[j] != slot(j);
+    mm[j] = __ballot(moved);
+    mo[j] = __ballot(moved && pos[j] >= kend);
+    if (lane == 0) {
+      s_cnt[0][j * NW + wv] = __builtin_popcountll(mm[j]);
+      s_cnt[1][j * NW + wv] = __builtin_popcountll(mo[j]);
+    }
+  }
+  __syncthreads();
+  int bns = 0, bnout = 0;
+  {
+    int *rec = ipiv + 2 * n + 1 + (size_t)(K0 / KB) * LU_PREC;
+    int *trec = ipiv + lu_trec_off(n, K0 / KB);
+    const unsigned long long before = (1ull << lane) - 1ull;
+    static_for<R>([&](auto js) {
+      constexpr int j = js;
+      int e = bns, o = bnout;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const int cm = s_cnt[0][j * NW + w], co = s_cnt[1][j * NW + w];
+        e += w < wv ? cm : 0;
+        o += w < wv ? co : 0;
+        bns += cm;
+        bnout += co;
       }
-      s_nout = no;
-      s_ns = ns;
-    }
-    __syncthreads();
-    const int bns = s_ns, bnout = s_nout;
-    {
-      // ---- the block's net interchanges: the record of the forward solves
-      // (read in pivot mode 1) and the trailing record of the update kernel
-      int *rec = ipiv + 2 * n + 1 + (size_t)(K0 / KB) * LU_PREC;
-      for (int e = t; e < bns; e += NT) { rec[1 + e] = s_srow[e]; rec[1 + 2 * KB + e] = s_sorig[e]; }
-      if (t == 0) rec[0] = bns;
-      int *trec = ipiv + lu_trec_off(n, K0 / KB);
-      for (int e = t; e < kb; e += NT) trec[1 + e] = s_topsrc[e];
-      for (int e = t; e < bnout; e += NT) { trec[1 + KB + e] = s_outrow[e]; trec[1 + 2 * KB + e] = s_outsrc[e]; }
-      if (t == 0) trec[0] = bnout;
-    }
-    // ---- left columns [0, K0) (pivot mode 0 only): move the touched rows,
-    // 16 columns at a time, through LDS (bns * 16 <= 2 KB * 16 = SU entries)
-    if (left && bns > 0 && K0 > 0) {
-      for (int c0 = 0; c0 < K0; c0 += 16) {
-        for (int e = t; e < bns * 16; e += NT) s_u[e] = A[(size_t)(c0 + e / bns) * lda + s_sorig[e % bns]];
-        __syncthreads();
-        for (int e = t; e < bns * 16; e += NT) A[(size_t)(c0 + e / bns) * lda + s_srow[e % bns]] = s_u[e];
-        __syncthreads();
-      }
-    }
-    // ---- X = inv(L11) (unit lower, zero outside kb x kb) in T arithmetic,
-    // column-major into this block's slot of the diagonal-block inverses
-    // (read by the triangular solves, and below by U12 = X A12).  Four lanes
-    // per column: lane q of column c keeps x[m] = X(4 m + q, c) in registers
-    // and sums the terms k = q (mod 4) of each substitution step; the sums meet
-    // by shuffles.  The strictly lower triangle of L11 is staged in s_u, packed
-    // by rows (row i at i (i - 1) / 2; 2016 entries), with zeros in rows and
-    // columns past kb.
-    C *X = blks + P.blk_off + (size_t)(K0 / KB) * KB * KB;
-    static_assert(KB * (KB - 1) / 2 <= SU, "packed L11 fits in s_u");
-    for (int e = t; e < KB * KB; e += NT) {
-      const int i = e % KB, k = e / KB;
-      if (k < i) {
-        const C v = A[(size_t)(K0 + k) * lda + K0 + (i < kb ? i : 0)];
-        s_u[i * (i - 1) / 2 + k] = (i < kb) ? v : czero<T>();
-      }
-    }
-    __syncthreads();
-    if (t < 4 * KB) {
-      const int c = t >> 2, q = t & 3;
-      C x[KB / 4];
-#pragma unroll
-      for (int m = 0; m < KB / 4; ++m) x[m] = czero<T>();
-#pragma unroll
-      for (int mi = 0; mi < KB / 4; ++mi) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = 4 * mi + r;
-          C s = czero<T>();
-#pragma unroll
-          for (int m = 0; m <= mi; ++m)     // entry (i, 4 m + q) of L11 when 4 m + q < i
-            s = cfma(s, (m < mi || q < r) ? s_u[i * (i - 1) / 2 + 4 * m + q] : czero<T>(), x[m]);
-          s.x += quad_xor1(s.x); s.y += quad_xor1(s.y);
-          s.x += quad_xor2(s.x); s.y += quad_xor2(s.y);
-          const C v = (i < c || i >= kb || c >= kb) ? czero<T>() : ((i == c) ? mk<T>(1, 0) : czero<T>() - s);
-          if (r == q) x[mi] = v;
+      const int row = slot(j);
+      if (pos[j] < kend) trec[1 + pos[j] - K0] = row;
+      if ((mm[j] >> lane) & 1ull) {
+        e += __builtin_popcountll(mm[j] & before);
+        s_srow[e] = pos[j];
+        s_sorig[e] = row;
+        rec[1 + e] = pos[j];
+        rec[1 + 2 * KB + e] = row;
+        if (pos[j] >= kend) {
+          o += __builtin_popcountll(mo[j] & before);
+          trec[1 + KB + o] = pos[j];
+          trec[1 + 2 * KB + o] = row;
         }
       }
+    });
+    if (t == 0) { rec[0] = bns; trec[0] = bnout; }
+  }
+  // ---- the block's rows into their final order, MC columns at a time: every
+  // moving row is read before any is written
+  constexpr int MC = 8;
+  for (int c0 = K0; c0 < kend; c0 += MC) {
+    T vx[R][MC], vy[R][MC];
 #pragma unroll
-      for (int m = 0; m < KB / 4; ++m) X[c * KB + 4 * m + q] = x[m];
-    }
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+      for (int c = 0; c < MC; ++c) {
+        const C v = at(c0 + c, slot(j));
+        vx[j][c] = v.x;
+        vy[j][c] = v.y;
+      }
     __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+      if ((mm[j] >> lane) & 1ull) {
+#pragma unroll
+        for (int c = 0; c < MC; ++c) at(c0 + c, pos[j]) = mk<T>(vx[j][c], vy[j][c]);
+      }
+  }
+  __syncthreads();
+  // ---- left columns [0, K0) (pivot mode 0 only): move the touched rows,
+  // 16 columns at a time, through LDS (bns * 16 <= 2 KB * 16 = SU entries)
+  if (left && bns > 0 && K0 > 0) {
+    for (int c0 = 0; c0 < K0; c0 += 16) {
+      for (int e = t; e < bns * 16; e += NT) s_u[e] = A[(size_t)(c0 + e / bns) * lda + s_sorig[e % bns]];
+      __syncthreads();
+      for (int e = t; e < bns * 16; e += NT) A[(size_t)(c0 + e / bns) * lda + s_srow[e % bns]] = s_u[e];
+      __syncthreads();
+    }
+  }
+  // ---- X = inv(L11) (unit lower, zero outside kb x kb) in T arithmetic,
+  // column-major into this block's slot of the diagonal-block inverses
+  // (read by the triangular solves, and below by U12 = X A12).  Four lanes
+  // per column: lane q of column c keeps x[m] = X(4 m + q, c) in registers
+  // and sums the terms k = q (mod 4) of each substitution step; the sums meet
+  // by shuffles.  The strictly lower triangle of L11 is staged in s_u, packed
+  // by rows (row i at i (i - 1) / 2; 2016 entries), with zeros in rows and
+  // columns past kb.
+  C *X = blks + P.blk_off + (size_t)(K0 / KB) * KB * KB;
+  static_assert(KB * (KB - 1) / 2 <= SU, "packed L11 fits in s_u");
+  for (int e = t; e < KB * KB; e += NT) {
+    const int i = e % KB, k = e / KB;
+    if (k < i) {
+      const C v = A[(size_t)(K0 + k) * lda + K0 + (i < kb ? i : 0)];
+      s_u[i * (i - 1) / 2 + k] = (i < kb) ? v : czero<T>();
+    }
+  }
+  __syncthreads();
+  if (t < 4 * KB) {
+    const int c = t >> 2, q = t & 3;
+    C x[KB / 4];
+#pragma unroll
+    for (int m = 0; m < KB / 4; ++m) x[m] = czero<T>();
+#pragma unroll
+    for (int mi = 0; mi < KB / 4; ++mi) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 4 * mi + r;
+        C s = czero<T>();
+#pragma unroll
+        for (int m = 0; m <= mi; ++m)     // entry (i, 4 m + q) of L11 when 4 m + q < i
+          s = cfma(s, (m < mi || q < r) ? s_u[i * (i - 1) / 2 + 4 * m + q] : czero<T>(), x[m]);
+        s.x += quad_xor1(s.x); s.y += quad_xor1(s.y);
+        s.x += quad_xor2(s.x); s.y += quad_xor2(s.y);
+        const C v = (i < c || i >= kb || c >= kb) ? czero<T>() : ((i == c) ? mk<T>(1, 0) : czero<T>() - s);
+        if (r == q) x[mi] = v;
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < KB / 4; ++m) X[c * KB + 4 * m + q] = x[m];
+  }
+  __syncthreads();
   // ---- final row permutation: row r of L U is row perm[r] of the input,
-  // composed in LDS (s_slot, idle now) by one thread, then stored; only the
-  // LAPACK form (pivot mode 0) has it: the mode-1 solves use the block records
-  static_assert(sizeof(s_u) >= 1280 * sizeof(int), "the pivots fit in s_u");
+  // composed in LDS by one thread, then stored; only the LAPACK form (pivot
+  // mode 0) has it: the mode-1 solves use the block records
+  static_assert(sizeof(s_u) >= 2 * 1280 * sizeof(int), "two row lists fit in s_u");
   if (left && kend == n) {
     int *perm = ipiv + n;
-    int *s_ip = reinterpret_cast<int *>(s_u);   // the pivots, read by one thread
+    int *s_ip = reinterpret_cast<int *>(s_u), *s_slot = s_ip + 1280;   // the pivots, the rows
     __syncthreads();
     for (int r = t; r < n; r += NT) { s_slot[r] = r; s_ip[r] = ipiv[r]; }
     __syncthreads();
@@ -533,7 +586,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 && NT
     info[pi] = myinfo;
     if (kend == n) ipiv[2 * n] = left ? 0 : 1;
   }
-  }  // block K0
 }
 
 
