@@ -135,10 +135,13 @@ template <typename T> __device__ inline cx<T> crecip(cx<T> b) {
 // rank-1 update.  With rows that moved at every pivot, serial net permutations
 // and strips of 16 columns loaded, updated and stored in turn, the panels of
 // one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.91
-// and 1.37 (256 such matrices: 1.88 and 2.92 ms, now 1.12 and 1.90); 0.38 and
-// 0.41 ms of that are the columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.
+// and 1.36 (256 such matrices: 1.88 and 2.92 ms, now 1.12 and 1.90); 0.38 and
+// 0.41 ms of that are the columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.  One row
+// per thread fits the registers of three waves per SIMD; two rows would spill
+// there, and run 2-4% faster in those of two (800 matrices of order 480: 2.69
+// and 2.64 ms in FP32, 5.15 and 4.93 in FP64).
 template <typename T, int NB, int NT, int R>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R <= 2 && NT == 256 ? 3 : 2))) void k_lu_panel(const PointDev *__restrict__ pts, cx<T> *__restrict__ mats,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT == 256 ? 3 : 2))) void k_lu_panel(const PointDev *__restrict__ pts, cx<T> *__restrict__ mats,
                                                  int *__restrict__ pivs, cx<T> *__restrict__ blks,
                                                  int *__restrict__ info, const int *__restrict__ order, int left,
                                                  int K0) {
