@@ -460,7 +460,7 @@ def main():
         })
         lu_ms = chosen["ms_lu_kernel"]
         achieved = chosen["lu_flops"] / (lu_ms * 1e-3) / 1e12
-        lu_kernel = ("FP32 batched complex LU: per 64-column block step k_lu_panel<float, 16, 256, R, 16> (R = 3 for "
+        lu_kernel = ("FP32 batched complex LU: per 64-column block step k_lu_panel<float, 16, 256, R> (R = 3 for "
                      "N = 128, 2 for N <= 96) and k_lu_trail<float> (matrix-core update), "
                      f"{chosen['lu_launches']} segments on concurrent streams; achieved = LU flops / span of the LU")
         out["roofline"] = {
