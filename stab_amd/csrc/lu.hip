@@ -134,8 +134,8 @@ template <typename T> __device__ inline cx<T> crecip(cx<T> b) {
 // columns, each an arg-max, a publication through LDS, one barrier and a
 // rank-1 update.  With rows that moved at every pivot, serial net permutations
 // and strips of 16 columns loaded, updated and stored in turn, the panels of
-// one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.91
-// and 1.36 (256 such matrices: 1.88 and 2.92 ms, now 1.12 and 1.90); 0.38 and
+// one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.86
+// and 1.35 (256 such matrices: 1.88 and 2.92 ms, now 1.01 and 1.83); 0.38 and
 // 0.41 ms of that are the columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.  One row
 // per thread fits the registers of three waves per SIMD; two rows would spill
 // there, and run 2-4% faster in those of two (800 matrices of order 480: 2.69
@@ -302,26 +302,33 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT
     const int c0 = k0 + NB, w = kend - c0;      // the rest of the block column
     if (w <= 0) break;
     // ---- A12: the pivot rows of the rest, staged by the waves after the
-    // first, while 16 (8) lanes of the first form inv(L11) (unit lower), one
-    // column per lane in registers, term k of every row as soon as x[k] is known
-    // (the terms k < c vanish: x[k] = 0 there)
+    // first, while the first forms inv(L11) (unit lower): four lanes per column
+    // c, lane q of them with the rows i = q (mod 4) in registers, term k of every
+    // row as soon as x[k] is known (the terms k < c vanish: x[k] = 0 there).  With
+    // a lane per column the panels took 1.12 and 1.90 ms (256 of order 480).
     if (wv == 0) {
-      if (lane < NB) {
-        const int c = lane;
-        C x[NB];
+      if (lane < 4 * NB) {
+        const int c = lane >> 2, q = lane & 3;
+        C x[NB / 4];
 #pragma unroll
-        for (int i = 0; i < NB; ++i) x[i] = mk<T>((T)(i == c), 0);
+        for (int m = 0; m < NB / 4; ++m) x[m] = mk<T>((T)(4 * m + q == c), 0);
         static_for<NB - 1>([&](auto ks) {
-          constexpr int k = ks;
-          x[k] = mk<T>(k < c ? (T)0 : x[k].x, k < c ? (T)0 : x[k].y);
+          constexpr int k = ks, mk_ = k / 4, qk = k % 4;
+          C xk = mk<T>(dpp_move<0x55 * qk>(x[mk_].x), dpp_move<0x55 * qk>(x[mk_].y));
+          xk = mk<T>(k < c ? (T)0 : xk.x, k < c ? (T)0 : xk.y);
 #pragma unroll
-          for (int i = k + 1; i < NB; ++i) {
-            const C l = s_blk[i * NB + k];
-            x[i] = cfms(x[i], mk<T>(k < c ? (T)0 : l.x, k < c ? (T)0 : l.y), x[k]);
+          for (int m = mk_; m < NB / 4; ++m) {
+            const C l = s_blk[(4 * m + q) * NB + k];
+            const C v = cfms(x[m], mk<T>(k < c ? (T)0 : l.x, k < c ? (T)0 : l.y), xk);
+            const bool up = m > mk_ || q > qk;          // rows below k only
+            x[m] = mk<T>(up ? v.x : x[m].x, up ? v.y : x[m].y);
           }
         });
 #pragma unroll
-        for (int i = 0; i < NB; ++i) s_linv[i * NB + c] = x[i];
+        for (int m = 0; m < NB / 4; ++m) {
+          const int i = 4 * m + q;
+          s_linv[i * NB + c] = mk<T>(i < c ? (T)0 : x[m].x, i < c ? (T)0 : x[m].y);
+        }
       }
     } else {
       for (int e = t - 64; e < NB * w; e += NT - 64) {
@@ -409,7 +416,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT
       });
     } else {
       // FP64 (and 512 threads, whose staging would not fit in s_u), on the VALU
-      // (the FP64 matrix cores give the same sums in 1.42 ms against 1.37):
+      // (the FP64 matrix cores give the same sums, 1.42 ms against 1.37):
       // G columns of a row at a time, the next group's entries loaded while one
       // is computed
       constexpr int G = 4;
