@@ -28,6 +28,7 @@
 // those of U.  With left = 1 (pivot mode 0, the LAPACK form) L is in final
 // row order and perm (ipiv + n, P as a row list) is stored too; with left = 0
 // the columns left of each block keep their rows (mode 1).
+#include "bounds.h"
 #include "common.h"
 #include <type_traits>
 #include <utility>
@@ -544,7 +545,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT
   for (int e = t; e < KB * KB; e += NT) {
     const int i = e % KB, k = e / KB;
     if (k < i) {
-      const C v = A[(size_t)(K0 + k) * lda + K0 + (i < kb ? i : 0)];
+      const C v = A[lu_l11_src(K0, kb, i, k, lda)];
       s_u[i * (i - 1) / 2 + k] = (i < kb) ? v : czero<T>();
     }
   }

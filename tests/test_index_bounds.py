@@ -1,0 +1,42 @@
+"""Index rules of the kernels (stab_amd/csrc/bounds.h), compiled with g++ and
+checked on the host over every size they meet."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+
+def _run(tmp_path, body):
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("g++ not available")
+    src, exe = tmp_path / "bounds.cpp", tmp_path / "bounds"
+    src.write_text('#include "bounds.h"\n#include <cstdio>\nint main() {\n  long long bad = 0;\n' + body +
+                   '  std::printf("%lld\\n", bad);\n  return 0;\n}\n')
+    r = subprocess.run([cxx, "-O1", "-std=c++17", "-I", os.path.join(ROOT, "stab_amd", "csrc"), str(src), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0
+    return int(out.stdout)
+
+
+def test_l11_staging_stays_in_the_matrix(tmp_path):
+    """Every order (multiples of 32 to 1280), every 64-column block, every
+    entry: the element read lies in the n x n matrix, and is entry (i, k) of
+    the block where the block has one."""
+    assert _run(tmp_path, r'''
+  for (int n = 32; n <= 1280; n += 32)
+    for (int K0 = 0; K0 < n; K0 += 64) {
+      const int kb = n - K0 < 64 ? n - K0 : 64;
+      for (int i = 0; i < 64; ++i)
+        for (int k = 0; k < i; ++k) {
+          const long long e = lu_l11_src(K0, kb, i, k, n);
+          bad += e < 0 || e >= (long long)n * n;
+          if (i < kb) bad += e != (long long)(K0 + k) * n + K0 + i;
+        }
+    }
+''') == 0
