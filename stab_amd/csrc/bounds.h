@@ -12,3 +12,14 @@
 constexpr long long lu_l11_src(int K0, int kb, int i, int k, int lda) {
   return (long long)(K0 + (i < kb ? k : 0)) * lda + K0 + (i < kb ? i : 0);
 }
+
+// Row that k_schur moves to position pos (pos < m <= 64) when it orders the
+// eigenvalues: the first lane of the ballot `at` of the lanes that hold the
+// largest modulus.  A lane outside [pos, m) carries -1 and no eigenvalue; with
+// NaN in every lane of the range (the factors of a singular matrix) the
+// maximum is that -1 and only such lanes are in the ballot, so they are masked
+// and pos stays where it is.
+constexpr int schur_pick(unsigned long long at, int pos, int m) {
+  at &= (m < 64 ? (1ull << m) - 1 : ~0ull) & ~((1ull << pos) - 1);
+  return at ? __builtin_ctzll(at) : pos;
+}

@@ -9,6 +9,7 @@
 //     u = L(sigma)^-1 (-C1 z1 - C2 (z2 + sigma z1)),  T z = [u; z1 + sigma u].
 // Solves use the LU factors (FP64, or equilibrated FP32 followed by FP64
 // iterative-refinement steps whose residuals use the matrix-free pencil).
+#include "bounds.h"
 #include "pencil.h"
 
 #define KS_MMAX 64
@@ -1062,8 +1063,7 @@ __global__ __launch_bounds__(128) void k_schur(const PointDev *__restrict__ pts,
       const double av = (lane >= pos && lane < m) ? sqrt(abs2(Hs[min(lane, m - 1) * LD + min(lane, m - 1)])) : -1.0;
       double bv = av;
       for (int off = 32; off > 0; off >>= 1) bv = fmax(bv, __shfl_xor(bv, off));
-      const unsigned long long at = __ballot(av == bv);
-      const int best = at ? max(pos, __builtin_ctzll(at)) : pos;   // NaN entries compare unequal
+      const int best = schur_pick(__ballot(av == bv), pos, m);      // a row of H whatever its entries
       Rot *rl = rot + (pos & 1) * m;
       const zd t22 = Hs[best * LD + best];                          // the eigenvalue that moves up
       for (int k = best - 1; k >= pos; --k) {

@@ -40,3 +40,36 @@ def test_l11_staging_stays_in_the_matrix(tmp_path):
         }
     }
 ''') == 0
+
+
+def test_schur_reorder_picks_a_row_of_the_matrix(tmp_path):
+    """The row brought to the front by k_schur, from the ballot its 64 lanes
+    form, over basis sizes, positions and patterns of NaN, infinite, equal and
+    ordinary moduli: inside [pos, m), the first of the largest, pos when every
+    modulus is NaN."""
+    assert _run(tmp_path, r'''
+  const double nan = __builtin_nan(""), inf = __builtin_inf();
+  unsigned s = 1;
+  for (int m = 2; m <= 64; ++m)
+    for (int pos = 0; pos < m; ++pos)
+      for (int pat = 0; pat < 12; ++pat) {
+        double av[64], bv = -1.0;
+        for (int l = 0; l < 64; ++l) {
+          s = s * 1664525u + 1013904223u;
+          const double r = (double)(s >> 8) / 16777216.0;
+          double v = pat == 0 ? nan : pat == 1 ? 0.0 : pat == 2 ? 1.0 : pat == 3 ? (r < 0.5 ? nan : 2.0) : r;
+          if (pat == 4 && r < 0.1) v = inf;
+          if (pat >= 8 && r < 0.9) v = nan;
+          av[l] = (l >= pos && l < m) ? v : -1.0;
+          if (av[l] > bv) bv = av[l];       // fmax drops NaN
+        }
+        unsigned long long at = 0;
+        int want = pos;
+        double wv = -1.0;
+        for (int l = 0; l < 64; ++l) at |= (unsigned long long)(av[l] == bv) << l;
+        for (int l = pos; l < m; ++l)
+          if (av[l] > wv) { wv = av[l]; want = l; }
+        const int got = schur_pick(at, pos, m);
+        bad += got < pos || got >= m || got != want;
+      }
+''') == 0
