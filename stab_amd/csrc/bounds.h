@@ -1,6 +1,7 @@
-// Index rules of kernels that have to stay in range for every size, free of
-// HIP types so they can be compiled and checked on the host (constexpr
-// functions are host and device functions alike).
+// Rules of kernels that have to hold for every size and value (indexes that
+// stay in range, NaN that is not lost), free of HIP types so they can be
+// compiled and checked on the host (constexpr functions are host and device
+// functions alike).
 #pragma once
 
 // Element of the matrix (column-major, leading dimension lda) that k_lu_panel
@@ -22,4 +23,12 @@ constexpr long long lu_l11_src(int K0, int kb, int i, int k, int lda) {
 constexpr int schur_pick(unsigned long long at, int pos, int m) {
   at &= (m < 64 ? (1ull << m) - 1 : ~0ull) & ~((1ull << pos) - 1);
   return at ? __builtin_ctzll(at) : pos;
+}
+
+// The largest of n residual estimates (none negative), NaN when any is: NaN
+// must not pass for the zero that fmax would leave of it.
+constexpr double est_max(const double *est, int n) {
+  double mx = 0.0;
+  for (int i = 0; i < n; ++i) mx = (est[i] > mx || est[i] != est[i]) ? est[i] : mx;
+  return mx;
 }

@@ -27,7 +27,7 @@
 struct KSState {
   int j0;        // first column to expand
   int k;         // kept columns after the last restart
-  int done;      // 1: every wanted pair converged; 2: stopped on stagnation
+  int done;      // 1: every wanted pair converged; 2: stopped on stagnation or NaN
   int cycles;
   double resmax; // max relative Ritz residual estimate of the wanted pairs
   double best;   // smallest resmax seen
@@ -1137,16 +1137,16 @@ __global__ __launch_bounds__(128) void k_schur(const PointDev *__restrict__ pts,
   }
   __syncthreads();
   if (t == 0) {
-    double mx = 0.0;
-    for (int i = 0; i < nev; ++i) mx = fmax(mx, s_est[i]);
+    const double mx = est_max(s_est, nev);
     S.resmax = mx;
     S.cycles += 1;
     if (S.cycles == 1 || mx < 0.1 * S.best) { S.best = fmin(mx, S.cycles == 1 ? mx : S.best); S.stall = 0; }
     else S.stall += 1;
     S.best = fmin(S.best, mx);
-    // converged, or no tenfold progress in three cycles (an ill-conditioned
-    // cluster among the wanted pairs): stop this point
-    S.done = (mx <= tol) ? 1 : ((S.stall >= 3) ? 2 : 0);
+    // converged; else stop this point on NaN (the factors of a singular matrix:
+    // nothing left to iterate) or without tenfold progress in three cycles (an
+    // ill-conditioned cluster among the wanted pairs)
+    S.done = (mx <= tol) ? 1 : ((mx != mx || S.stall >= 3) ? 2 : 0);
     st[blockIdx.x] = S;
   }
 }
@@ -1386,16 +1386,16 @@ __global__ __launch_bounds__(64) void k_schur_seq(const PointDev *__restrict__ p
   }
   __syncthreads();
   if (t == 0) {
-    double mx = 0.0;
-    for (int i = 0; i < nev; ++i) mx = fmax(mx, s_est[i]);
+    const double mx = est_max(s_est, nev);
     S.resmax = mx;
     S.cycles += 1;
     if (S.cycles == 1 || mx < 0.1 * S.best) { S.best = fmin(mx, S.cycles == 1 ? mx : S.best); S.stall = 0; }
     else S.stall += 1;
     S.best = fmin(S.best, mx);
-    // converged, or no tenfold progress in three cycles (an ill-conditioned
-    // cluster among the wanted pairs): stop this point
-    S.done = (mx <= tol) ? 1 : ((S.stall >= 3) ? 2 : 0);
+    // converged; else stop this point on NaN (the factors of a singular matrix:
+    // nothing left to iterate) or without tenfold progress in three cycles (an
+    // ill-conditioned cluster among the wanted pairs)
+    S.done = (mx <= tol) ? 1 : ((mx != mx || S.stall >= 3) ? 2 : 0);
     st[blockIdx.x] = S;
   }
 }

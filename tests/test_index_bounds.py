@@ -1,5 +1,5 @@
-"""Index rules of the kernels (stab_amd/csrc/bounds.h), compiled with g++ and
-checked on the host over every size they meet."""
+"""Rules of the kernels (stab_amd/csrc/bounds.h), compiled with g++ and checked
+on the host over the sizes and values they meet."""
 import os
 import shutil
 import subprocess
@@ -72,4 +72,28 @@ def test_schur_reorder_picks_a_row_of_the_matrix(tmp_path):
         const int got = schur_pick(at, pos, m);
         bad += got < pos || got >= m || got != want;
       }
+''') == 0
+
+
+def test_residual_estimate_keeps_nan(tmp_path):
+    """The largest estimate of the wanted pairs: the plain maximum of numbers
+    and infinities, NaN (neither converged nor a number to improve on) with a
+    NaN in any place."""
+    assert _run(tmp_path, r'''
+  const double nan = __builtin_nan(""), inf = __builtin_inf();
+  for (int n = 1; n <= 16; ++n) {
+    double e[16];
+    for (int i = 0; i < n; ++i) e[i] = 1e-14 * (i + 1);
+    bad += est_max(e, n) != 1e-14 * n;
+    for (int k = 0; k < n; ++k) {
+      const double was = e[k];
+      e[k] = inf;
+      bad += est_max(e, n) != inf;
+      e[k] = nan;
+      bad += est_max(e, n) <= 1e-12 || est_max(e, n) > 1e-12;
+      e[k] = was;
+    }
+    for (int i = 0; i < n; ++i) e[i] = nan;
+    bad += est_max(e, n) <= 1e-12 || est_max(e, n) > 1e-12;
+  }
 ''') == 0
