@@ -609,7 +609,9 @@ template <typename T, int NB>
 int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max, int &nconv, double &ms_arnoldi) {
   bool any_spatial = false;
   for (const auto &d : B.h) any_spatial |= (d.itype == 2);
-  const int full = (kp.ir != 0 || any_spatial) ? 1 : 0;
+  // FP32 factors are those of the equilibrated pencil; the full operator undoes
+  // the scales, with refinement steps (ir != 0) or without
+  const int full = (sizeof(T) == 4 || kp.ir != 0 || any_spatial) ? 1 : 0;
   const size_t lds = op_lds_bytes(B.npadmax, B.nymax, 1, B.nvecmax);
   const size_t lds_arn = op_lds_bytes(B.npadmax, B.nymax, full, B.nvecmax);
   if (lds > 160 * 1024) return fail(c, STAB_E_ARG, "operator workspace %zu B exceeds LDS", lds);
@@ -630,17 +632,16 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
                          B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax, B.nymax, B.nvecmax,
                          cyc == 0 ? 1 : 0);
     };
-    if (sizeof(T) == 8 && kp.track) {
-      if constexpr (sizeof(T) == 8) {
-        if (full) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
-        else arnoldi(k_arnoldi<T, NB, WIDE_NT, false, true>);
-      }
-    } else if (full) {
+    if constexpr (sizeof(T) == 8) {
+      if (kp.track && full) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
+      else if (kp.track) arnoldi(k_arnoldi<T, NB, WIDE_NT, false, true>);
+      else if (full && wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
+      else if (full) arnoldi(k_arnoldi<T, NB, 256, true>);
+      else if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, false>);
+      else arnoldi(k_arnoldi<T, NB, 256, false>);
+    } else {
       if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
       else arnoldi(k_arnoldi<T, NB, 256, true>);
-    } else if constexpr (sizeof(T) == 8) {        // FP32 factors come with refinement, the full operator
-      if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, false>);
-      else arnoldi(k_arnoldi<T, NB, 256, false>);
     }
     HIPCHECK(c, hipEventRecord(c->ev[6], c->stream));
     hipLaunchKernelGGL(kp.track ? k_schur_seq : k_schur, dim3(npts), dim3(kp.track ? 64 : 128), lds_schur, c->stream, B.pts,
