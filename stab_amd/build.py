@@ -9,7 +9,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SRC = os.path.join(HERE, "csrc", "api.hip")
 OUT = os.path.join(HERE, "libstab_hip.so")
-DEPS = ("api.hip", "prep.hip", "assemble.hip", "lu.hip", "eig.hip", "pencil.h", "common.h", "bounds.h")
+DEPS = ("api.hip", "prep.hip", "assemble.hip", "lu.hip", "eig.hip", "pencil.h", "common.h", "bounds.h", "mlp_bufs.h")
 
 HIPCC_FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

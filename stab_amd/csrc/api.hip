@@ -7,6 +7,7 @@
 #include "eig.hip"
 #include "mlp.hip"
 #include "lu_plan.h"
+#include "mlp_bufs.h"
 
 #include <algorithm>
 #include <cmath>
@@ -702,84 +703,36 @@ struct stab_mlp {
   stab_ctx *c = nullptr;
   MlpNet net;
   int np = 0, t = 0;
-  float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr, *scl = nullptr, *loss = nullptr;
+  float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr, *scl = nullptr;
   int *meta = nullptr;                 // parameter segments (k_mlp_init), then
   int *tiles = nullptr;                // the 16 x 16 weight tiles of k_mlp_grad
   int ntile = 0;
-  int hist_cap = 0;
-  int cap_b = 0;                       // rows of the batch buffers (k_mlp_rows)
-  short *actT = nullptr, *dzT = nullptr;
-  float *act32 = nullptr, *part = nullptr, *losspart = nullptr;
-  int cap_n = 0;                       // rows of the data set buffers
-  float *Xall = nullptr, *Tall = nullptr, *xraw = nullptr, *traw = nullptr;
   float *hx = nullptr;                 // pinned rows of stab_mlp_predict: cap_h inputs, then cap_h outputs
   int cap_h = 0;
-  std::vector<void *> owned;
+  DevPool pool;
+  MlpRowBufs rows;
+  MlpSetBufs set;
+  MlpLossBuf loss;
 };
 
 namespace {
 
-int mlp_alloc(stab_mlp *M, size_t bytes, void **out) {
-  void *q = nullptr;
-  HIPCHECK(M->c, hipMalloc(&q, bytes ? bytes : 16));
-  M->owned.push_back(q);
-  *out = q;
-  return STAB_OK;
-}
-
-template <typename P>
-int mlp_get(stab_mlp *M, size_t bytes, P **out) {
-  void *q;
-  int rc = mlp_alloc(M, bytes, &q);
-  *out = (P *)q;
-  return rc;
-}
-
-void mlp_free(stab_mlp *M, void *q) {
-  if (!q) return;
-  (void)hipFree(q);
-  for (auto &o : M->owned)
-    if (o == q) o = nullptr;
-}
-
 // Work buffers for batches of up to B rows (B a multiple of 16).
 int mlp_reserve(stab_mlp *M, int B) {
-  if (B <= M->cap_b) return STAB_OK;
-  mlp_free(M, M->actT); mlp_free(M, M->dzT); mlp_free(M, M->act32); mlp_free(M, M->part); mlp_free(M, M->losspart);
-  M->cap_b = 0;
-  int rc;
-  const size_t hid = (size_t)M->net.depth * M->net.width;
-  if ((rc = mlp_get(M, sizeof(short) * (M->net.nin_p + hid) * B, &M->actT)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(short) * (hid + 16) * B, &M->dzT)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * hid * B, &M->act32)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * (hid + 16) * (B / 16), &M->part)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * (B / 16), &M->losspart)) != STAB_OK) return rc;
-  M->cap_b = B;
-  return STAB_OK;
-}
-
-int mlp_reserve_data(stab_mlp *M, int n) {
-  if (n <= M->cap_n) return STAB_OK;
-  mlp_free(M, M->Xall); mlp_free(M, M->Tall); mlp_free(M, M->xraw); mlp_free(M, M->traw);
-  M->cap_n = 0;
-  int rc;
-  if ((rc = mlp_get(M, sizeof(float) * (size_t)n * M->net.nin_p, &M->Xall)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * (size_t)n * M->net.nout, &M->Tall)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * (size_t)n * M->net.nin, &M->xraw)) != STAB_OK) return rc;
-  if ((rc = mlp_get(M, sizeof(float) * (size_t)n * M->net.nout, &M->traw)) != STAB_OK) return rc;
-  M->cap_n = n;
+  HIPCHECK(M->c, M->rows.reserve(M->pool, M->net.nin_p, (size_t)M->net.depth * M->net.width, B));
   return STAB_OK;
 }
 
 // Loss and gradient (grad != nullptr) or one Adam step over a batch of B rows
-// of the n normalised rows in Xall, Tall: two launches.
+// of the n normalised rows in set.X, set.T: two launches.
 void mlp_step(stab_mlp *M, int n, int B, uint64_t seed, int step, float *grad, float lr, int hist_slot) {
   hipStream_t s = M->c->stream;
+  const MlpRowBufs &R = M->rows;
   const int ncol = M->net.depth * M->net.width + 16;
-  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(B / 16), dim3(MLP_T), 0, s, M->net, M->p, M->scl, M->Xall, (float *)nullptr, n,
-                     B, M->Tall, (unsigned long long)seed, step, M->actT, M->dzT, M->act32, M->part, M->losspart);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(M->ntile + (ncol + 63) / 64), dim3(64), 0, s, M->net, B, M->ntile, M->tiles, M->dzT,
-                     M->actT, M->part, M->losspart, grad, M->p, M->m, M->v, lr, M->t, M->loss, hist_slot);
+  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(B / 16), dim3(MLP_T), 0, s, M->net, M->p, M->scl, M->set.X, (float *)nullptr, n,
+                     B, M->set.T, (unsigned long long)seed, step, R.actT, R.dzT, R.act32, R.part, R.losspart);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(M->ntile + (ncol + 63) / 64), dim3(64), 0, s, M->net, B, M->ntile, M->tiles, R.dzT,
+                     R.actT, R.part, R.losspart, grad, M->p, M->m, M->v, lr, M->t, M->loss.p, hist_slot);
 }
 
 int mlp_check_rows(stab_mlp *M, int n) {
@@ -1695,18 +1648,21 @@ int stab_mlp_create(stab_ctx *c, int nin, int width, int depth, int nout, uint64
   M->np = off;
   int rc;
   auto bail = [&](int code) { stab_mlp_destroy(M); return code; };
-  if ((rc = mlp_get(M, sizeof(float) * M->np, &M->p)) != STAB_OK) return bail(rc);
-  if ((rc = mlp_get(M, sizeof(float) * M->np, &M->g)) != STAB_OK) return bail(rc);
-  if ((rc = mlp_get(M, sizeof(float) * M->np, &M->m)) != STAB_OK) return bail(rc);
-  if ((rc = mlp_get(M, sizeof(float) * M->np, &M->v)) != STAB_OK) return bail(rc);
-  if ((rc = mlp_get(M, sizeof(float) * (2 * N.nin_p + 32), &M->scl)) != STAB_OK) return bail(rc);
+  auto get = [&](size_t bytes, auto *&out) -> int {
+    HIPCHECK(c, M->pool.get(bytes, out));
+    return STAB_OK;
+  };
+  if ((rc = get(sizeof(float) * M->np, M->p)) != STAB_OK) return bail(rc);
+  if ((rc = get(sizeof(float) * M->np, M->g)) != STAB_OK) return bail(rc);
+  if ((rc = get(sizeof(float) * M->np, M->m)) != STAB_OK) return bail(rc);
+  if ((rc = get(sizeof(float) * M->np, M->v)) != STAB_OK) return bail(rc);
+  if ((rc = get(sizeof(float) * (2 * N.nin_p + 32), M->scl)) != STAB_OK) return bail(rc);
   const int nseg = (int)(meta.size() / 6);
   M->ntile = (int)(tiles.size() / 4);
   meta.insert(meta.end(), tiles.begin(), tiles.end());
-  if ((rc = mlp_get(M, sizeof(int) * meta.size(), &M->meta)) != STAB_OK) return bail(rc);
+  if ((rc = get(sizeof(int) * meta.size(), M->meta)) != STAB_OK) return bail(rc);
   M->tiles = M->meta + 6 * nseg;
-  M->hist_cap = 0;
-  if ((rc = mlp_get(M, sizeof(float), &M->loss)) != STAB_OK) return bail(rc);
+  if (M->loss.reserve(M->pool, 0) != hipSuccess) return bail(fail(c, STAB_E_HIP, "allocation of the network's loss failed"));
   std::vector<float> scl(2 * N.nin_p + 32, 0.f);
   for (int i = 0; i < N.nin_p; ++i) scl[N.nin_p + i] = 1.f;
   for (int o = 0; o < 16; ++o) scl[2 * N.nin_p + 16 + o] = 1.f;
@@ -1723,8 +1679,7 @@ int stab_mlp_create(stab_ctx *c, int nin, int width, int depth, int nout, uint64
 
 int stab_mlp_destroy(stab_mlp *M) {
   if (!M) return STAB_OK;
-  for (void *q : M->owned)
-    if (q) (void)hipFree(q);
+  M->pool.clear();
   if (M->hx) (void)hipHostFree(M->hx);
   delete M;
   return STAB_OK;
@@ -1777,6 +1732,7 @@ int stab_mlp_predict(stab_mlp *M, int n, const float *x, float *y) {
     while (cap < want) cap *= 2;
     if (hipHostMalloc((void **)&M->hx, sizeof(float) * (size_t)cap * (nin + nout), hipHostMallocDefault) != hipSuccess) {
       M->hx = nullptr;
+      (void)hipGetLastError();
       return fail(M->c, STAB_E_NOMEM, "pinned allocation of %d prediction rows failed", cap);
     }
     M->cap_h = cap;
@@ -1795,16 +1751,15 @@ int stab_mlp_predict(stab_mlp *M, int n, const float *x, float *y) {
   return STAB_OK;
 }
 
-// Upload n rows and targets and normalise them into Xall, Tall.
+// Upload n rows and targets and normalise them into set.X, set.T.
 static int mlp_upload(stab_mlp *M, int n, const float *x, const float *t) {
-  int rc;
-  if ((rc = mlp_reserve_data(M, n)) != STAB_OK) return rc;
   hipStream_t s = M->c->stream;
   const MlpNet &N = M->net;
-  HIPCHECK(M->c, hipMemcpyAsync(M->xraw, x, sizeof(float) * (size_t)n * N.nin, hipMemcpyHostToDevice, s));
-  HIPCHECK(M->c, hipMemcpyAsync(M->traw, t, sizeof(float) * (size_t)n * N.nout, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_mlp_normalize, dim3(n), dim3(64), 0, s, N.nin, N.nin_p, N.nout, M->xraw, M->traw, M->scl, M->Xall,
-                     M->Tall);
+  MlpSetBufs &D = M->set;
+  HIPCHECK(M->c, D.reserve(M->pool, N.nin, N.nin_p, N.nout, n));
+  HIPCHECK(M->c, hipMemcpyAsync(D.xraw, x, sizeof(float) * (size_t)n * N.nin, hipMemcpyHostToDevice, s));
+  HIPCHECK(M->c, hipMemcpyAsync(D.traw, t, sizeof(float) * (size_t)n * N.nout, hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_mlp_normalize, dim3(n), dim3(64), 0, s, N.nin, N.nin_p, N.nout, D.xraw, D.traw, M->scl, D.X, D.T);
   return STAB_OK;
 }
 
@@ -1817,7 +1772,7 @@ int stab_mlp_loss_grad(stab_mlp *M, int n, const float *x, const float *t, float
   if ((rc = mlp_upload(M, n, x, t)) != STAB_OK) return rc;
   mlp_step(M, n, n, 0, 0, M->g, 0.f, -1);
   HIPCHECK(M->c, hipGetLastError());
-  if (loss) HIPCHECK(M->c, hipMemcpyAsync(loss, M->loss, sizeof(float), hipMemcpyDeviceToHost, M->c->stream));
+  if (loss) HIPCHECK(M->c, hipMemcpyAsync(loss, M->loss.p, sizeof(float), hipMemcpyDeviceToHost, M->c->stream));
   if (grad) HIPCHECK(M->c, hipMemcpyAsync(grad, M->g, sizeof(float) * M->np, hipMemcpyDeviceToHost, M->c->stream));
   HIPCHECK(M->c, hipStreamSynchronize(M->c->stream));
   return STAB_OK;
@@ -1831,13 +1786,7 @@ int stab_mlp_train(stab_mlp *M, int n, const float *x, const float *t, int batch
   if (n < batch) return fail(M->c, STAB_E_ARG, "MLP training set (%d rows) smaller than the batch (%d)", n, batch);
   HIPCHECK(M->c, hipSetDevice(M->c->device));
   if ((rc = mlp_reserve(M, batch)) != STAB_OK) return rc;
-  if (loss_hist && steps > M->hist_cap) {
-    mlp_free(M, M->loss);
-    M->loss = nullptr;
-    M->hist_cap = 0;
-    if ((rc = mlp_get(M, sizeof(float) * (size_t)(steps + 1), &M->loss)) != STAB_OK) return rc;
-    M->hist_cap = steps;
-  }
+  if (loss_hist) HIPCHECK(M->c, M->loss.reserve(M->pool, steps));
   hipStream_t s = M->c->stream;
   if ((rc = mlp_upload(M, n, x, t)) != STAB_OK) return rc;
   for (int st = 0; st < steps; ++st) {
@@ -1846,7 +1795,7 @@ int stab_mlp_train(stab_mlp *M, int n, const float *x, const float *t, int batch
   }
   HIPCHECK(M->c, hipGetLastError());
   if (loss_hist)
-    HIPCHECK(M->c, hipMemcpyAsync(loss_hist, M->loss + 1, sizeof(float) * steps, hipMemcpyDeviceToHost, s));
+    HIPCHECK(M->c, hipMemcpyAsync(loss_hist, M->loss.p + 1, sizeof(float) * steps, hipMemcpyDeviceToHost, s));
   HIPCHECK(M->c, hipStreamSynchronize(s));
   return STAB_OK;
 }
