@@ -593,10 +593,15 @@ int run_graph(stab_ctx *c, const std::vector<long long> &sig, F issue, int *how)
 // `active` points: one wide work-group per point while that leaves CUs without
 // any (lu_solve_wide), four waves beyond, where two or three work-groups share
 // a CU and memory is the bound.  STAB_WIDE_POINTS moves the line.
-// Krylov leading modes, N = 96, four waves against wide, ms: 14.1 / 11.1 at 64
-// points, 23.6 / 20.1 at 256, 32.5 / 27.4 at 320, 27.1 / 26.3 at 512, 51.3 /
-// 50.4 at 1024; inverse iteration 7.1 / 6.8 at 64, 7.1 / 7.1 at 256, 8.3 / 8.6
-// at 320, 15.1 / 15.3 at 1024.
+// Four waves against wide, ms, at N = 128 and 1 / 16 / 64 / 256 points: Krylov
+// in FP64, temporal 10.3 / 14.3 / 15.4 / 25.1 and 7.6 / 10.1 / 13.2 / 24.2;
+// Krylov on FP32 factors, spatial 58 / 67 / 73 / 97 and 39 / 43 / 48 / 78;
+// inverse iteration on FP32 factors 3.2 / 3.9 / 4.4 / 6.3 and 3.0 / 3.5 / 4.0 /
+// 6.1, on FP64 factors 3.7 / 4.3 / 5.0 / 9.2 and 3.7 / 4.2 / 5.4 / 9.5 (the
+// fallback of a missed point gains more than that loses).  At N = 96 the two
+// meet for inverse iteration at 256 points (8.3 / 8.6 at 320); Krylov in FP64
+// still gains beyond (32.5 / 27.4 at 320, 27.1 / 26.3 at 512, 51.3 / 50.4 at
+// 1024).
 constexpr int WIDE_NT = 512;
 bool wide_points(int active) { return active <= env_int("STAB_WIDE_POINTS", 256); }
 
@@ -608,8 +613,8 @@ struct KSParams {
 
 template <typename T, int NB>
 int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max, int &nconv, double &ms_arnoldi) {
-  bool any_spatial = false;
-  for (const auto &d : B.h) any_spatial |= (d.itype == 2);
+  bool any_spatial = false, any_temporal = false;
+  for (const auto &d : B.h) { any_spatial |= (d.itype == 2); any_temporal |= (d.itype == 1); }
   // FP32 factors are those of the equilibrated pencil; the full operator undoes
   // the scales, with refinement steps (ir != 0) or without
   const int full = (sizeof(T) == 4 || kp.ir != 0 || any_spatial) ? 1 : 0;
@@ -624,17 +629,24 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
   std::vector<KSState> hs(npts);
   cycles_max = 0;
   ms_arnoldi = 0.0;
+  // Temporal points under the full operator (FP32 factors, or FP64 beside
+  // spatial points) stay at four waves: in the wide kernel their shifted solve
+  // is out of line, with every access a flat one.  N = 128, four waves against
+  // wide: FP32 40 / 59 / 63 / 88 ms and 64 / 97 / 109 / 173 at 1 / 16 / 64 / 256
+  // points; FP64 with spatial points 21 and 28 ms at 64 + 1, 33 and 42 at 128 + 128.
+  const bool keep4 = full && any_temporal;
   int active = npts;        // points that have not stopped
   for (int cyc = 0; cyc < kp.maxcycles; ++cyc) {
     HIPCHECK(c, hipEventRecord(c->ev[5], c->stream));
-    const bool wide = kp.track || wide_points(active);
+    const bool wide = (kp.track || wide_points(active)) && !keep4;
     auto arnoldi = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(npts), dim3(wide ? WIDE_NT : 256), lds_arn, c->stream, B.pts, mats, B.pivs, blks,
                          B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax, B.nymax, B.nvecmax,
                          cyc == 0 ? 1 : 0);
     };
     if constexpr (sizeof(T) == 8) {
-      if (kp.track && full) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
+      if (kp.track && full && wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
+      else if (kp.track && full) arnoldi(k_arnoldi<T, NB, 256, true, true>);
       else if (kp.track) arnoldi(k_arnoldi<T, NB, WIDE_NT, false, true>);
       else if (full && wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
       else if (full) arnoldi(k_arnoldi<T, NB, 256, true>);
