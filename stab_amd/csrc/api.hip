@@ -741,7 +741,7 @@ void mlp_step(stab_mlp *M, int n, int B, uint64_t seed, int step, float *grad, f
   hipStream_t s = M->c->stream;
   const MlpRowBufs &R = M->rows;
   const int ncol = M->net.depth * M->net.width + 16;
-  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(B / 16), dim3(MLP_T), 0, s, M->net, M->p, M->scl, M->set.X, (float *)nullptr, n,
+  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(B / 16), dim3(mlp_threads(M->net)), 0, s, M->net, M->p, M->scl, M->set.X, (float *)nullptr, n,
                      B, M->set.T, (unsigned long long)seed, step, R.actT, R.dzT, R.act32, R.part, R.losspart);
   hipLaunchKernelGGL(k_mlp_grad, dim3(M->ntile + (ncol + 63) / 64), dim3(64), 0, s, M->net, B, M->ntile, M->tiles, R.dzT,
                      R.actT, R.part, R.losspart, grad, M->p, M->m, M->v, lr, M->t, M->loss.p, hist_slot);
@@ -1753,7 +1753,7 @@ int stab_mlp_predict(stab_mlp *M, int n, const float *x, float *y) {
   for (int r0 = 0; r0 < n; r0 += CH) {
     const int rows = std::min(CH, n - r0);
     memcpy(M->hx, x + (size_t)r0 * nin, sizeof(float) * (size_t)rows * nin);
-    hipLaunchKernelGGL(k_mlp_rows<false>, dim3((rows + 15) / 16), dim3(MLP_T), 0, M->c->stream, M->net, M->p, M->scl,
+    hipLaunchKernelGGL(k_mlp_rows<false>, dim3((rows + 15) / 16), dim3(mlp_threads(M->net)), 0, M->c->stream, M->net, M->p, M->scl,
                        (const float *)M->hx, hy, rows, rows, (const float *)nullptr, 0ull, 0, (short *)nullptr,
                        (short *)nullptr, (float *)nullptr, (float *)nullptr, (float *)nullptr);
     HIPCHECK(M->c, hipGetLastError());

@@ -14,9 +14,9 @@
 // its dependent phases, not by arithmetic: per-layer GEMM launches with their
 // own gather, bias-sum, loss and Adam launches took 649 us a step at batch
 // 1024 and width 128 (of which 490 us the bias sums, one thread walking the
-// batch), these two 30 us.  A prediction
-// of 8191 rows at width 256 went from 411 to 60 us, of 12 rows from 72 to 26 us
-// (pinned host rows read and written in place, one launch, one wait).
+// batch), these two 28 us.  A prediction of 8191 rows at width 256 went from
+// 411 to 42 us, of 12 rows from 72 to 24 us (pinned host rows read and
+// written in place, one launch, one wait).
 //
 // Flat parameter layout (FP32), dimensions padded to multiples of 16
 // (nin_p = pad16(nin), nout_p = pad16(nout); padded rows/columns stay zero):
@@ -25,7 +25,7 @@
 //   W_o [nout_p x width], b_o [nout_p]
 // W is row-major by output unit: W[o * in + i].
 #include "common.h"
-
+#include <algorithm>
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -36,7 +36,7 @@ __device__ inline short to_bf16(float x) {
   return (short)(u >> 16);
 }
 
-#define MLP_T 512        // eight waves per 16-row tile: one 16-column tile each at width 128
+#define MLP_T 1024       // most threads of a 16-row tile (mlp_threads)
 #define MLP_WMAX 512     // widest layer
 #define MLP_LMAX 9       // 8 hidden layers and the output layer
 #define MLP_KU 8         // depth-16 steps whose operands are loaded together
@@ -46,6 +46,16 @@ struct MlpNet {
   int nin, nin_p, width, depth, nout, nout_p;
   int off_w[MLP_LMAX], off_b[MLP_LMAX];
 };
+
+// Threads of k_mlp_rows: a wave per 16-column tile of a layer, eight to sixteen.
+// A batch of few rows runs on few CUs, each reading every weight (1 MB a layer
+// at width 512) through its own memory path, so bytes in flight per CU are
+// what counts.  64 inputs, width 512, eight layers: 16 rows took 244 us with
+// eight waves and the weights by operand order, where one launch per layer
+// over all CUs had taken 181; 187 with the loads along rows, 119 with sixteen
+// waves too (a step of 16 rows 402, 308, 344, 248).  Width 256, three layers:
+// 36, 80, 29, 26.
+inline int mlp_threads(const MlpNet &N) { return std::min(MLP_T, std::max(512, 4 * N.width)); }
 
 __device__ inline unsigned mlp_hash(unsigned long long seed, unsigned a, unsigned b) {
   unsigned long long h = seed ^ (0x9E3779B97F4A7C15ull * (a + 1)) ^ (0xC2B2AE3D27D4EB4Full * (b + 7));
@@ -60,22 +70,27 @@ __device__ inline unsigned mlp_hash(unsigned long long seed, unsigned a, unsigne
 // A[l % 16][k0 + 4 (l / 16) + j] and W(k0 + 4 (l / 16) + j, n0 + l % 16), j < 4;
 // accumulator register i is entry (4 (l / 16) + i, l % 16).  The weights of
 // MLP_KU steps are loaded before the first is used, from clamped in-range
-// steps, so a pass costs one memory latency per 128 of K.
+// steps, so a pass costs one memory latency per 128 of K.  In the forward
+// product four consecutive lanes load 64 consecutive bytes of a weight row
+// (lane l row l / 4) and the BF16 values change lanes afterwards; with the
+// rows on consecutive lanes, as the operand has them, a load of the wave met
+// sixteen rows and a CU took in some 15 bytes a cycle.
 template <bool TRANS>
 __device__ inline f32x4 mlp_tile(const short (*__restrict__ A)[MLP_WMAX + 8], int K, const float *__restrict__ w, int ldn,
                                  int n0) {
   const int l = threadIdx.x & 63, r = l & 15, q = 4 * (l >> 4);
+  const int from = 4 * (4 * r + (l >> 4));           // byte index of the lane that loaded this lane's weights
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int kb = 0; kb < K; kb += 16 * MLP_KU) {
     f32x4 wv[MLP_KU];
 #pragma unroll
     for (int s = 0; s < MLP_KU; ++s) {
-      const int k = min(kb + 16 * s, K - 16) + q;
+      const int k = min(kb + 16 * s, K - 16);
       if (TRANS) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) wv[s][j] = w[(size_t)(k + j) * ldn + n0 + r];
+        for (int j = 0; j < 4; ++j) wv[s][j] = w[(size_t)(k + q + j) * ldn + n0 + r];
       } else {
-        wv[s] = *(const f32x4 *)(w + (size_t)(n0 + r) * ldn + k);
+        wv[s] = *(const f32x4 *)(w + (size_t)(n0 + (l >> 2)) * ldn + k + 4 * (l & 3));
       }
     }
 #pragma unroll
@@ -86,6 +101,13 @@ __device__ inline f32x4 mlp_tile(const short (*__restrict__ A)[MLP_WMAX + 8], in
         bf16x4 b;
 #pragma unroll
         for (int j = 0; j < 4; ++j) b[j] = to_bf16(wv[s][j]);
+        if (!TRANS) {
+          union { bf16x4 h; int d[2]; } u;
+          u.h = b;
+          u.d[0] = __builtin_amdgcn_ds_bpermute(from, u.d[0]);
+          u.d[1] = __builtin_amdgcn_ds_bpermute(from, u.d[1]);
+          b = u.h;
+        }
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
       }
     }
@@ -119,14 +141,14 @@ __global__ __launch_bounds__(MLP_T) void k_mlp_rows(MlpNet N, const float *__res
                                                     float *__restrict__ losspart) {
   __shared__ __align__(16) short s_a[2][16][MLP_WMAX + 8];   // 8 shorts of padding: rows start on different banks
   __shared__ int s_src[16];
-  constexpr int NW = MLP_T / 64;
+  const int NT = blockDim.x, NW = NT / 64;
   const int t = threadIdx.x, w = t >> 6, l = t & 63, r = l & 15, q = 4 * (l >> 4);
   const int b0 = blockIdx.x * 16, W = N.width, L = N.depth;
   if (TRAIN) {
     if (t < 16) s_src[t] = (B == n) ? b0 + t : (int)(mlp_hash(seed, (unsigned)step, (unsigned)(b0 + t)) % (unsigned)n);
     __syncthreads();
   }
-  for (int e = t; e < 16 * N.nin_p; e += MLP_T) {
+  for (int e = t; e < 16 * N.nin_p; e += NT) {
     const int row = e / N.nin_p, i = e - row * N.nin_p;
     float v = 0.f;
     if (TRAIN) v = x[(size_t)s_src[row] * N.nin_p + i];
