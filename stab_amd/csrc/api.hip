@@ -597,11 +597,10 @@ int run_graph(stab_ctx *c, const std::vector<long long> &sig, F issue, int *how)
 // in FP64, temporal 10.3 / 14.3 / 15.4 / 25.1 and 7.6 / 10.1 / 13.2 / 24.2;
 // Krylov on FP32 factors, spatial 58 / 67 / 73 / 97 and 39 / 43 / 48 / 78;
 // inverse iteration on FP32 factors 3.2 / 3.9 / 4.4 / 6.3 and 3.0 / 3.5 / 4.0 /
-// 6.1, on FP64 factors 3.7 / 4.3 / 5.0 / 9.2 and 3.7 / 4.2 / 5.4 / 9.5 (the
-// fallback of a missed point gains more than that loses).  At N = 96 the two
-// meet for inverse iteration at 256 points (8.3 / 8.6 at 320); Krylov in FP64
-// still gains beyond (32.5 / 27.4 at 320, 27.1 / 26.3 at 512, 51.3 / 50.4 at
-// 1024).
+// 6.1; inverse iteration on FP64 factors 3.7 / 4.3 / 5.0 / 9.2 and 3.7 / 4.2 /
+// 5.4 / 9.5, so it stays at four waves (lead_invit).  At N = 96 the two meet
+// for inverse iteration at 256 points (8.3 / 8.6 at 320); Krylov in FP64 still
+// gains beyond (32.5 / 27.4 at 320, 27.1 / 26.3 at 512, 51.3 / 50.4 at 1024).
 constexpr int WIDE_NT = 512;
 bool wide_points(int active) { return active <= env_int("STAB_WIDE_POINTS", 256); }
 
@@ -1337,7 +1336,9 @@ static int lead_invit(stab_ctx *c, int npts, const stab_point *pts, int mode, in
   // points' first passes, instead of in a second launch whose few work-groups
   // leave the GPU idle; it needs only 2 NT more LDS entries, as it reuses the
   // first pass's vectors.  STAB_FUSE2=0 issues k_invit2 after k_invit.
-  const bool wide = wide_points(npts);
+  // FP64 factors stay at four waves: the wide kernel would spill 154 registers
+  // of the second pass and took as long or longer at every size (wide_points)
+  const bool wide = f32 && wide_points(npts);
   const size_t lds_f = lds + (wide ? 0 : sizeof(zd) * 2 * 256);   // a wide work-group has tmp for two right-hand sides
   const bool fuse2 = env_int("STAB_FUSE2", 1) && lds_f <= 160 * 1024;
   const bool do2 = fuse2 || lds2 <= 160 * 1024;
@@ -1383,9 +1384,8 @@ static int lead_invit(stab_ctx *c, int npts, const stab_point *pts, int mode, in
     };
     const zf *mf = (const zf *)B.mats;
     const zd *md = (const zd *)B.mats;
-    if (f32 && wide) invit(k_invit<float, 16, WIDE_NT>, mf);
+    if (wide) invit(k_invit<float, 16, WIDE_NT>, mf);
     else if (f32) invit(k_invit<float, 16, 256>, mf);
-    else if (wide) invit(k_invit<double, 16, WIDE_NT>, md);
     else invit(k_invit<double, 16, 256>, md);
     HIPCHECK(c, hipGetLastError());
     if ((rc2 = mark(4)) != STAB_OK) return rc2;
