@@ -194,12 +194,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT
   // row j of this thread (rows past the matrix: row K0), and its entry in a
   // column.  The column's address is uniform and passes through the asm so that
   // it stays a scalar of its own: 2 R NB whole addresses per lane, kept from the
-  // loads to the stores, would spill.
+  // loads to the stores, would spill.  The asm takes it as a global address: a
+  // generic one comes back without its address space, and the accesses become
+  // flat ones, which also count as LDS accesses where the wave waits.
   auto slot = [&](int j) { return K0 + t + j * NT < n ? K0 + t + j * NT : K0; };
   auto at = [&](int col, unsigned row) -> C & {
-    char *cp = reinterpret_cast<char *>(A + (size_t)col * lda);
+    typedef __attribute__((address_space(1))) char gchar;
+    gchar *cp = (gchar *)(A + (size_t)col * lda);
     asm volatile("" : "+s"(cp));
-    return *reinterpret_cast<C *>(cp + row * (unsigned)sizeof(C));
+    return *(C *)(cp + row * (unsigned)sizeof(C));
   };
   for (int k0 = K0; k0 < kend; k0 += NB) {
     // ---- load the panel (rows that were pivots earlier carry values that are
