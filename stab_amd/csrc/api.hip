@@ -637,23 +637,23 @@ int run_eig(stab_ctx *c, int npts, Batch &B, const KSParams &kp, int &cycles_max
   int active = npts;        // points that have not stopped
   for (int cyc = 0; cyc < kp.maxcycles; ++cyc) {
     HIPCHECK(c, hipEventRecord(c->ev[5], c->stream));
-    const bool wide = (kp.track || wide_points(active)) && !keep4;
+    const bool wide = wide_points(active) && !keep4;
     auto arnoldi = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(npts), dim3(wide ? WIDE_NT : 256), lds_arn, c->stream, B.pts, mats, B.pivs, blks,
                          B.scales, B.coef, B.ops, B.V, B.small, B.state, kp.m, kp.ir, B.npadmax, B.nymax, B.nvecmax,
                          cyc == 0 ? 1 : 0);
     };
+    auto by_width = [&](auto wide_kernel, auto four_waves) {
+      if (wide) arnoldi(wide_kernel);
+      else arnoldi(four_waves);
+    };
     if constexpr (sizeof(T) == 8) {
-      if (kp.track && full && wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true, true>);
-      else if (kp.track && full) arnoldi(k_arnoldi<T, NB, 256, true, true>);
-      else if (kp.track) arnoldi(k_arnoldi<T, NB, WIDE_NT, false, true>);
-      else if (full && wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
-      else if (full) arnoldi(k_arnoldi<T, NB, 256, true>);
-      else if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, false>);
-      else arnoldi(k_arnoldi<T, NB, 256, false>);
+      if (kp.track && full) by_width(k_arnoldi<T, NB, WIDE_NT, true, true>, k_arnoldi<T, NB, 256, true, true>);
+      else if (kp.track) by_width(k_arnoldi<T, NB, WIDE_NT, false, true>, k_arnoldi<T, NB, 256, false, true>);
+      else if (full) by_width(k_arnoldi<T, NB, WIDE_NT, true>, k_arnoldi<T, NB, 256, true>);
+      else by_width(k_arnoldi<T, NB, WIDE_NT, false>, k_arnoldi<T, NB, 256, false>);
     } else {
-      if (wide) arnoldi(k_arnoldi<T, NB, WIDE_NT, true>);
-      else arnoldi(k_arnoldi<T, NB, 256, true>);
+      by_width(k_arnoldi<T, NB, WIDE_NT, true>, k_arnoldi<T, NB, 256, true>);
     }
     HIPCHECK(c, hipEventRecord(c->ev[6], c->stream));
     hipLaunchKernelGGL(kp.track ? k_schur_seq : k_schur, dim3(npts), dim3(kp.track ? 64 : 128), lds_schur, c->stream, B.pts,

@@ -2,7 +2,7 @@
 sum is formed in an order that does not depend on the work-group (Gram-Schmidt
 coefficients by one wave each, norms by the first 256 threads), so the Krylov
 pairs, vectors and residuals are compared as they are, in both modes, and so is
-the inverse iteration with its Krylov fallback.  Every batch has to hold
+the inverse iteration with its Krylov fallback, tracked and not.  Every batch has to hold
 converged pairs and directly solved points, or nothing would be compared."""
 import numpy as np
 import pytest
@@ -24,8 +24,9 @@ def test_wide_is_bitwise_the_same(gpu_solver, monkeypatch, batch):
         for mode in (_lib.MODE_PLAIN_F64, _lib.MODE_MIXED):
             # near shifts are solved directly; the points' own shifts, one step only, leave the fallback to do it
             out[wide].append(gpu_solver.solve_leading(pts, mode, _lib.LEAD_INVIT, maxit=20, shifts=shifts, want_vectors=True))
-            out[wide].append(gpu_solver.solve_leading(pts, mode, _lib.LEAD_INVIT, maxit=1, want_vectors=True,
-                                                      shifts=[1.2 * s for s in shifts], fallback_shifts=shifts))
+            for method in (_lib.LEAD_INVIT, _lib.TRACK):
+                out[wide].append(gpu_solver.solve_leading(pts, mode, method, maxit=1, want_vectors=True,
+                                                          shifts=[1.2 * s for s in shifts], fallback_shifts=shifts))
     a, b = out["0"], out["1000000"]
     for x, y in zip(a[:2], b[:2]):
         assert np.array_equal(x.info, y.info) and np.array_equal(x.evals, y.evals) and np.array_equal(x.resid, y.resid)
@@ -33,6 +34,7 @@ def test_wide_is_bitwise_the_same(gpu_solver, monkeypatch, batch):
     for x, y in zip(a[2:], b[2:]):
         assert np.array_equal(x["info"], y["info"]) and np.array_equal(x["evals"], y["evals"])
         assert all(np.array_equal(u, v) for u, v in zip(x["evecs"], y["evecs"]))
-    for near, far in ((a[2], a[3]), (a[4], a[5])):
+    for near, far, tracked in (a[2:5], a[5:8]):
         assert np.any(near["info"] == _lib.INFO_OK)
         assert np.any(far["info"] == _lib.INFO_FALLBACK)
+        assert np.any(tracked["info"] == _lib.INFO_FALLBACK)
