@@ -283,7 +283,10 @@ __device__ inline double wave_sum(double x) {
 //   * NT / 4 row groups x 64 columns are in flight at once, and every register
 //     of a pass is reloaded, as soon as it is used, with the entry of the next
 //     pass, across block steps too: the loads of a step do not depend on the
-//     solution, so they arrive while the step before is finished;
+//     solution, so they are on their way while the step before is finished.
+//     The compiled loop waits for all of them, and for those of the inverse,
+//     issued last, at the head of each pass, so part of a memory latency is
+//     still met in every pass;
 //   * the same holds for the entries of the diagonal-block inverse (four waves,
 //     its quarters on the DPP rows, no partial sums in LDS) and for the
 //     interchange record (one entry per thread);
@@ -1160,6 +1163,8 @@ __global__ __launch_bounds__(128) void k_schur(const PointDev *__restrict__ pts,
 // with the sums of k_schur in the fallback, 1 of 25 tracked batches returned
 // other codes.  So the fallback of a tracked point keeps this order of
 // operations; it is rare (a quarter of 16-curve batches have such a point).
+// It costs such a point 2.95 ms a cycle (m = 40) where k_schur takes 1.21, and
+// 37 us a Gram-Schmidt step (n = 480) where the other form takes 14.
 // ---------------------------------------------------------------------------
 __device__ inline void givens_seq(zd x, zd y, double &c, zd &s) {
   const double ax = cabs(x), ay = cabs(y);
@@ -1685,9 +1690,10 @@ __host__ __device__ inline bool lead2_competes(int want, double alpha_r, zd sigm
 }
 
 // The second pass for point p (P = its descriptor), x1 holding the first
-// pass's vector (getevec normalisation) on entry.  x1, x2, a1, a2 and tmp2
-// (2 NT entries) are LDS; b1 and b2, read only by the lane that wrote them,
-// may be global.  L supplies the solve's scratch (y, rhs, tmp, w2), the
+// pass's vector (getevec normalisation) on entry.  x1, x2, a1, a2 and tmp2 (2
+// NT entries with 256 threads, 128 with more) are LDS; b1 and b2 may be
+// global: the products that write them end in a barrier, and the sums that
+// read them, whose stride (RT) is not the work-group's, come after it.  L supplies the solve's scratch (y, rhs, tmp, w2), the
 // products' (X1, X2, red) and nothing else, so x1 .. a2 may alias L.z, L.res,
 // L.y and L.rhs as long as a1, a2 are not L.rhs, L.y before the first step's
 // solve is done (they are written only inside the loop).

@@ -135,12 +135,13 @@ template <typename T> __device__ inline cx<T> crecip(cx<T> b) {
 // columns, each an arg-max, a publication through LDS, one barrier and a
 // rank-1 update.  With rows that moved at every pivot, serial net permutations
 // and strips of 16 columns loaded, updated and stored in turn, the panels of
-// one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.86
-// and 1.35 (256 such matrices: 1.88 and 2.92 ms, now 1.01 and 1.83); 0.38 and
-// 0.41 ms of that are the columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.  One row
-// per thread fits the registers of three waves per SIMD; two rows would spill
-// there, and run 2-4% faster in those of two (800 matrices of order 480: 2.69
-// and 2.64 ms in FP32, 5.15 and 4.93 in FP64).
+// one matrix of order 480 took 1.65 ms in FP32 and 2.34 ms in FP64, now 0.82
+// and 1.17 (256 such matrices: 1.88 and 2.92 ms, now 0.91 and 1.46).  While the
+// accesses were flat ones (0.86 and 1.35 ms; see `at`) 0.38 and 0.41 ms were the
+// columns, 0.17 and 0.55 A22, 0.11 and 0.12 X.  One row per thread fits the
+// registers of three waves per SIMD; two rows would spill there, and ran 2-4%
+// faster in those of two (800 matrices of order 480, flat accesses: 2.69 and
+// 2.64 ms in FP32, 5.15 and 4.93 in FP64).
 template <typename T, int NB, int NT, int R>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT == 256 ? 3 : 2))) void k_lu_panel(const PointDev *__restrict__ pts, cx<T> *__restrict__ mats,
                                                  int *__restrict__ pivs, cx<T> *__restrict__ blks,
@@ -420,9 +421,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(R == 1 && NT
       });
     } else {
       // FP64 (and 512 threads, whose staging would not fit in s_u), on the VALU
-      // (the FP64 matrix cores give the same sums, 1.42 ms against 1.37):
-      // G columns of a row at a time, the next group's entries loaded while one
-      // is computed
+      // (the FP64 matrix cores gave the same sums, 1.42 ms against 1.37 on flat
+      // accesses): G columns of a row at a time, the next group's entries loaded
+      // while one is computed
       constexpr int G = 4;
       static_for<R>([&](auto js) {
         constexpr int j = js;
