@@ -36,6 +36,9 @@ def test_nonfinite_point_is_not_solved(gpu_solver, ny):
         print(f"nonfinite N {ny} mode {mode}: lu", flush=True)
         lu, perm, dr, dc, info = gpu_solver.lu_factors(bad, mode)
         assert sorted(perm) == list(range(lu.shape[0]))
+        # a column that is NaN from its diagonal down had no candidate: the pivot stayed on the diagonal
+        nan = np.isnan(lu.real) | np.isnan(lu.imag)
+        assert any(nan[k:, k].all() for k in range(lu.shape[0] - 1))
         print(f"nonfinite N {ny} mode {mode}: solve", flush=True)
         r, alone = gpu_solver.solve([good, bad, good], mode), gpu_solver.solve([good], mode)
         assert r.info[1] in (_lib.INFO_NOCONV, _lib.INFO_SINGULAR)
